@@ -2,9 +2,10 @@
 //
 // Replaces the dense Matrix transform (fastmat/Matrix.pyx:1831-1842,
 // 1924-1935: ndarray.dot) for the dense factors of a Kron product
-// (Kron.pyx:267-341) and for plain dense matrices.
+// (Kron.pyx:267-341) and for plain dense matrices.  Plain products beyond
+// 128 x 128 and those in float64 / complex128 are in fm_gemm_direct.hpp.
 //
-// One kernel computes Y[i, c] = sum_l A_eff[i, l] * Bm[l, c] with strided
+// The strided kernels here compute Y[i, c] = sum_l A_eff[i, l] * Bm[l, c] with strided
 // addressing:
 //   A_eff[i, l] = A[i*a_rs + l*a_cs]                  (transpose by strides)
 //   Bm[l, c]    = X[s*(o*bos + l*brs + j*bjs) + p]    c -> (o, j, p)
@@ -18,9 +19,11 @@
 // Tiling: 256 threads (4 wave64) own a 64 x 64 output tile; each wave owns a
 // 32 x 32 quarter as 2 x 2 MFMA 16x16 blocks; K advances in slabs of 16
 // staged through LDS.
+#include <algorithm>
 #include <type_traits>
 
 #include "fm_common.hpp"
+#include "fm_gemm_direct.hpp"
 
 namespace fm {
 
@@ -40,8 +43,6 @@ struct GemmArgs {
 };
 
 constexpr int GT_M = 64, GT_N = 64, GT_K = 16;
-
-static fm_status gemm_launch_tiled(const GemmArgs &g, hipStream_t stream);
 
 __device__ __forceinline__ int64_t col_base(const GemmArgs &g, int64_t c, int64_t os, int64_t js,
                                             int *part) {
@@ -277,39 +278,12 @@ static int64_t max_offset(const GemmArgs &g, int64_t os, int64_t rs, int64_t js,
 }
 
 // ----------------------------------------------- other element types
-// Y = A X (adjoint: A^H X) for int8/16/32/64, float64 and complex128 data of
-// one type (ndarray.dot of the promoted operands, Matrix.pyx:1842, 1935).
-// Integers accumulate in 64-bit unsigned arithmetic and are truncated to the
-// element width at the store: the same residue modulo 2^bits as numpy's
-// integer dot, which sums in a 64-bit integer and casts the sum to the
-// output type.  float64 / complex128 accumulate in FP64.  Tiles of 64 rows x
+// Y = A X (adjoint: A^T X) for int8/16/32/64 data of one type (ndarray.dot
+// of the promoted operands, Matrix.pyx:1842, 1935).  Sums run in 64-bit
+// unsigned arithmetic and are truncated to the element width at the store:
+// the same residue modulo 2^bits as numpy's integer dot, which sums in a
+// 64-bit integer and casts the sum to the output type.  Tiles of 64 rows x
 // 16 columns of Y per 256-thread workgroup, K in LDS slabs of 32.
-template <typename T> struct GenAcc { typedef T type; };
-template <> struct GenAcc<int8_t> { typedef uint64_t type; };
-template <> struct GenAcc<int16_t> { typedef uint64_t type; };
-template <> struct GenAcc<int32_t> { typedef uint64_t type; };
-template <> struct GenAcc<int64_t> { typedef uint64_t type; };
-
-template <typename T> __device__ __forceinline__ typename GenAcc<T>::type gen_widen(T v) {
-    if constexpr (std::is_integral<T>::value) return uint64_t(int64_t(v));
-    else return v;
-}
-template <typename T> __device__ __forceinline__ T gen_conj(T v) { return v; }
-template <> __device__ __forceinline__ cpx<double> gen_conj(cpx<double> v) { return conj(v); }
-template <typename A> __device__ __forceinline__ A gen_mac(A acc, A a, A b) { return acc + a * b; }
-template <>
-__device__ __forceinline__ cpx<double> gen_mac(cpx<double> acc, cpx<double> a, cpx<double> b) {
-    return acc + cmul(a, b);
-}
-template <typename T> __device__ __forceinline__ T gen_narrow(typename GenAcc<T>::type v) {
-    if constexpr (std::is_integral<T>::value) return T(v);  // modulo 2^bits
-    else return v;
-}
-template <typename T> __device__ __forceinline__ typename GenAcc<T>::type gen_zero() {
-    if constexpr (std::is_same<T, cpx<double>>::value) return mk(0.0, 0.0);
-    else return typename GenAcc<T>::type(0);
-}
-
 constexpr int GG_M = 64, GG_J = 16, GG_K = 32;
 
 template <typename T>
@@ -318,7 +292,7 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(int64_t M, int64_t K,
                                                            int adjoint, const T *__restrict__ X,
                                                            int64_t ldx, T *__restrict__ Y,
                                                            int64_t ldy) {
-    typedef typename GenAcc<T>::type Acc;
+    typedef uint64_t Acc;
     __shared__ Acc sa[GG_K][GG_M + 1];
     __shared__ Acc sx[GG_J][GG_K + 1];
     const int t = threadIdx.x;
@@ -327,28 +301,28 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(int64_t M, int64_t K,
     const int jl = (t >> 6) * 4;  // four columns per thread
     Acc acc[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) acc[q] = gen_zero<T>();
+    for (int q = 0; q < 4; ++q) acc[q] = 0;
     for (int64_t l0 = 0; l0 < K; l0 += GG_K) {
         // A slab: rows i0.., columns l0.. of A_eff (A or A^H)
         for (int e = t; e < GG_M * GG_K; e += 256) {
             const int ii = e % GG_M, ll = e / GG_M;
             const int64_t i = i0 + ii, l = l0 + ll;
-            Acc v = gen_zero<T>();
+            Acc v = 0;
             if (i < M && l < K)
-                v = adjoint ? gen_widen(gen_conj(A[l * lda + i])) : gen_widen(A[i * lda + l]);
+                v = Acc(int64_t(adjoint ? A[l * lda + i] : A[i * lda + l]));
             sa[ll][ii] = v;
         }
         for (int e = t; e < GG_J * GG_K; e += 256) {
             const int ll = e % GG_K, jj = e / GG_K;
             const int64_t l = l0 + ll, j = j0 + jj;
-            sx[jj][ll] = (l < K && j < k) ? gen_widen(X[j * ldx + l]) : gen_zero<T>();
+            sx[jj][ll] = (l < K && j < k) ? Acc(int64_t(X[j * ldx + l])) : 0;
         }
         __syncthreads();
 #pragma unroll 4
         for (int ll = 0; ll < GG_K; ++ll) {
             const Acc a = sa[ll][il];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) acc[q] = gen_mac(acc[q], a, sx[jl + q][ll]);
+            for (int q = 0; q < 4; ++q) acc[q] += a * sx[jl + q][ll];
         }
         __syncthreads();
     }
@@ -357,7 +331,7 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(int64_t M, int64_t K,
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const int64_t j = j0 + jl + q;
-        if (j < k) Y[j * ldy + i] = gen_narrow<T>(acc[q]);
+        if (j < k) Y[j * ldy + i] = T(acc[q]);  // modulo 2^bits
     }
 }
 
@@ -380,49 +354,148 @@ static fm_status gemm_generic(int adjoint, int64_t m, int64_t n, const void *A, 
     return FM_SUCCESS;
 }
 
-static fm_status dense_generic(int dtype, int adjoint, int64_t m, int64_t n, const void *A,
-                               int64_t lda, const void *x, int64_t ldx, void *y, int64_t ldy,
-                               int64_t k, hipStream_t s) {
-    switch (dtype) {
-    case FM_INT8: return gemm_generic<int8_t>(adjoint, m, n, A, lda, x, ldx, y, ldy, k, s);
-    case FM_INT16: return gemm_generic<int16_t>(adjoint, m, n, A, lda, x, ldx, y, ldy, k, s);
-    case FM_INT32: return gemm_generic<int32_t>(adjoint, m, n, A, lda, x, ldx, y, ldy, k, s);
-    case FM_INT64: return gemm_generic<int64_t>(adjoint, m, n, A, lda, x, ldx, y, ldy, k, s);
-    case FM_FLOAT64: return gemm_generic<double>(adjoint, m, n, A, lda, x, ldx, y, ldy, k, s);
-    case FM_COMPLEX128:
-        return gemm_generic<cpx<double>>(adjoint, m, n, A, lda, x, ldx, y, ldy, k, s);
-    default: break;
-    }
-    set_error("dense apply: unsupported element type %d", dtype);
-    return FM_ERR_TYPE;
+// ------------------------------------------------ direct-operand products
+static int cu_count() {
+    int dev = 0, ncu = 256;
+    if (hipGetDevice(&dev) == hipSuccess)
+        (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+    return ncu;
 }
 
-static fm_status gemm_launch(const GemmArgs &g, hipStream_t stream) {
-    const bool small = g.M <= SK_K && g.K <= SK_K && g.NC > 0 &&
-                       max_offset(g, g.bos, g.brs, g.bjs, g.K) < (int64_t(1) << 31) &&
-                       max_offset(g, g.yos, g.yrs, g.yjs, g.M) < (int64_t(1) << 31);
-    if (small) {
-        const int64_t tiles = ceil_div(g.NC, SK_N);
-        if (tiles == 0) return FM_SUCCESS;
-        int dev = 0, ncu = 256;
-        if (hipGetDevice(&dev) == hipSuccess)
-            (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-        // one workgroup fits a CU (A in registers: ~180 VGPRs, 2 waves per
-        // SIMD), so the grid is one workgroup per CU walking its tiles
-        static const int per_cu = knob("FASTMAT_AMD_SMALLK_WG_PER_CU", 1);
-        int64_t grid = int64_t(ncu) * (per_cu >= 1 && per_cu <= 4 ? per_cu : 1);
-        if (grid > tiles) grid = tiles;
-        ProfToken tok;
-        prof_begin(stream, &tok);
-        hipLaunchKernelGGL(gemm_smallk_kernel, dim3(unsigned(grid)), dim3(SK_T), 0, stream, g);
-        FM_CHECK_LAUNCH();
-        if (tok.active) {
-            const double bytes = 4.0 * (double(g.M) * g.K + double(g.K) * g.NC + double(g.M) * g.NC);
-            prof_end(stream, &tok, "gemm_smallk_kernel", bytes, 2.0 * double(g.M) * g.K * g.NC);
-        }
-        return FM_SUCCESS;
+template <typename S, bool XC, bool AK, int FM, int FN, int WM, int WN, int WK,
+          typename Off = uint32_t>
+static fm_status direct_launch(const DirectArgs<S> &g, hipStream_t stream) {
+    constexpr int TM = 16 * FM * WM, TN = (XC ? 8 : 16) * FN * WN;
+    constexpr size_t lds = WK > 1 ? size_t(WM) * WN * WK * FN * 4 * FM * 64 * sizeof(S) : 0;
+    static_assert(lds <= 64 * 1024, "K split's partial sums");
+    const int64_t tiles = ceil_div(g.M, TM) * ceil_div(g.NC, TN);
+    FM_REQUIRE(tiles < (int64_t(1) << 31), FM_ERR_VALUE, "dense product too large for one launch");
+    ProfToken tok;
+    prof_begin(stream, &tok);
+    hipLaunchKernelGGL((gemm_direct_kernel<S, Off, XC, AK, FM, FN, WM, WN, WK>), dim3(unsigned(tiles)),
+                       dim3(64 * WM * WN * WK), lds, stream, g);
+    FM_CHECK_LAUNCH();
+    if (tok.active) {
+        const double e = double(sizeof(S)), xs = XC ? 2.0 : 1.0;
+        const double mul = std::is_same<S, cpx<double>>::value ? 8.0 : 2.0;
+        prof_end(stream, &tok, "gemm_direct_kernel",
+                 e * (double(g.M) * g.K + xs * (double(g.K) + double(g.M)) * g.NC),
+                 mul * xs * double(g.M) * g.K * g.NC);
     }
-    return gemm_launch_tiled(g, stream);
+    return FM_SUCCESS;
+}
+
+// Tile shape of one product.  A workgroup's time goes with its tile's area
+// over K and a CU's with the tiles it gets, so cost = tiles per CU (rounded
+// up) x area x a factor for the smaller shapes' extra operand traffic per
+// MFMA.  The factors are measured times of every shape (us, M x K x NC,
+// one MI355X; A by rows / transposed product):
+//   float32     128x128  64x64  64x32  64x16  16x16   tiled kernel before
+//   2048x3072x1024  265    115    135    215    340   393
+//   3072x2048x1024  178    137    111    128    269   393 (transposed)
+//   4096x4096x4096 1075   1125   1352   2233   3569
+//   1000x777x130     65     18     11    7.7    7.9
+//   2500x2500x1     193     48     28     17    6.8
+//   float64      128x64  64x32  32x16  16x16
+//   2500x2500x1000  335    269    460    569
+//   1000x777x130     54     17     14     14
+//   complex128    64x64  32x32  16x16                 generic kernel before
+//   2500x2500x1000  897    778   1211
+//   1000x777x130    100     29     26                 171
+struct DirectShapeCost {
+    int64_t M, NC;
+    int ncu;
+    double operator()(int tm, int tn, double factor) const {
+        const int64_t tiles = ceil_div(M, tm) * ceil_div(NC, tn);
+        return double(ceil_div(tiles, ncu)) * tm * tn * factor;
+    }
+};
+
+template <typename S, bool XC, bool AK>
+static fm_status direct_pick(const DirectArgs<S> &g, hipStream_t stream) {
+    const DirectShapeCost cost{g.M, g.NC, cu_count()};
+    constexpr int X2 = XC ? 2 : 1;  // a complex column is two fragments
+    // a wave's rows and columns (at most 64) within 4 GiB of its first ones
+    // take 32-bit lane offsets; matrices beyond that the general addressing
+    const double reach = double(sizeof(S)) * (double(g.lda) * (AK ? std::min<int64_t>(g.M, 64) : 16) +
+                                              64.0);
+    const double xreach = double(sizeof(S)) * X2 * (double(g.ldx) * std::min<int64_t>(g.NC, 64) + 64.0);
+    if (reach >= 4294967296.0 || xreach >= 4294967296.0)
+        return direct_launch<S, XC, AK, 1, X2, 1, 1, 8, uint64_t>(g, stream);
+    if constexpr (XC) {
+        const double a = 2 * cost(128, 64, 1.0), b = 2 * cost(64, 32, AK ? 1.05 : 1.1),
+                     e = 2 * cost(64, 16, AK ? 1.2 : 1.03), d = 2 * cost(16, 16, 2.4);
+        if (a <= b && a <= e && a <= d) return direct_launch<S, XC, AK, 4, 4, 2, 2, 1>(g, stream);
+        if (b <= e && b <= d) return direct_launch<S, XC, AK, 4, 4, 1, 1, 4>(g, stream);
+        if (e <= d) return direct_launch<S, XC, AK, 4, 2, 1, 1, 8>(g, stream);
+        return direct_launch<S, XC, AK, 1, 2, 1, 1, 16>(g, stream);
+    } else if constexpr (std::is_same<S, float>::value) {
+        const double a = cost(128, 128, 1.0), b = cost(64, 64, AK ? 1.05 : 1.1),
+                     e = cost(64, 32, AK ? 1.2 : 1.03), c = cost(64, 16, AK ? 1.9 : 1.45),
+                     d = cost(16, 16, 2.8);
+        if (a <= b && a <= e && a <= c && a <= d)
+            return direct_launch<S, XC, AK, 4, 4, 2, 2, 1>(g, stream);
+        if (b <= e && b <= c && b <= d) return direct_launch<S, XC, AK, 4, 4, 1, 1, 4>(g, stream);
+        if (e <= c && e <= d) return direct_launch<S, XC, AK, 4, 2, 1, 1, 4>(g, stream);
+        if (c <= d) return direct_launch<S, XC, AK, 4, 1, 1, 1, 8>(g, stream);
+        return direct_launch<S, XC, AK, 1, 1, 1, 1, 16>(g, stream);
+    } else if constexpr (std::is_same<S, double>::value) {
+        const double a = cost(128, 64, 1.0), b = cost(64, 32, 1.0), c = cost(32, 16, 1.6),
+                     d = cost(16, 16, 2.1);
+        if (a <= b && a <= c && a <= d) return direct_launch<S, XC, AK, 4, 2, 2, 2, 1>(g, stream);
+        if (b <= c && b <= d) return direct_launch<S, XC, AK, 4, 2, 1, 1, 4>(g, stream);
+        if (c <= d) return direct_launch<S, XC, AK, 2, 1, 1, 1, 8>(g, stream);
+        return direct_launch<S, XC, AK, 1, 1, 1, 1, 16>(g, stream);
+    } else {
+        const double a = cost(64, 64, 1.0), b = cost(32, 32, 1.03), c = cost(16, 16, 1.25);
+        if (a <= b && a <= c) return direct_launch<S, XC, AK, 2, 2, 2, 2, 1>(g, stream);
+        if (b <= c) return direct_launch<S, XC, AK, 2, 2, 1, 1, 4>(g, stream);
+        return direct_launch<S, XC, AK, 1, 1, 1, 1, 8>(g, stream);
+    }
+}
+
+template <typename S, bool XC>
+static fm_status dense_direct(int adjoint, int64_t m, int64_t n, const void *A, int64_t lda,
+                              const void *x, int64_t ldx, void *y, int64_t ldy, int64_t k,
+                              hipStream_t s) {
+    DirectArgs<S> g;
+    g.M = adjoint ? n : m;
+    g.K = adjoint ? m : n;
+    g.NC = k;
+    g.A = (const S *)A;
+    g.lda = lda;
+    g.X = (const S *)x;
+    g.ldx = ldx;
+    g.Y = (S *)y;
+    g.ldy = ldy;
+    g.conj_a = adjoint;
+    if (adjoint) return direct_pick<S, XC, false>(g, s);
+    return direct_pick<S, XC, true>(g, s);
+}
+
+// Products that run on gemm_smallk_kernel.
+static bool gemm_is_small(const GemmArgs &g) {
+    return g.M <= SK_K && g.K <= SK_K && g.NC > 0 &&
+           max_offset(g, g.bos, g.brs, g.bjs, g.K) < (int64_t(1) << 31) &&
+           max_offset(g, g.yos, g.yrs, g.yjs, g.M) < (int64_t(1) << 31);
+}
+
+static fm_status gemm_launch_small(const GemmArgs &g, hipStream_t stream) {
+    const int64_t tiles = ceil_div(g.NC, SK_N);
+    // one workgroup fits a CU (A in registers: ~180 VGPRs, 2 waves per
+    // SIMD), so the grid is one workgroup per CU walking its tiles
+    static const int per_cu = knob("FASTMAT_AMD_SMALLK_WG_PER_CU", 1);
+    int64_t grid = int64_t(cu_count()) * (per_cu >= 1 && per_cu <= 4 ? per_cu : 1);
+    if (grid > tiles) grid = tiles;
+    ProfToken tok;
+    prof_begin(stream, &tok);
+    hipLaunchKernelGGL(gemm_smallk_kernel, dim3(unsigned(grid)), dim3(SK_T), 0, stream, g);
+    FM_CHECK_LAUNCH();
+    if (tok.active) {
+        const double bytes = 4.0 * (double(g.M) * g.K + double(g.K) * g.NC + double(g.M) * g.NC);
+        prof_end(stream, &tok, "gemm_smallk_kernel", bytes, 2.0 * double(g.M) * g.K * g.NC);
+    }
+    return FM_SUCCESS;
 }
 
 static fm_status gemm_launch_tiled(const GemmArgs &g, hipStream_t stream) {
@@ -463,8 +536,17 @@ extern "C" fm_status fm_dense_apply(int a_dtype, int x_dtype, int adjoint, int64
     FM_REQUIRE(A && x && y, FM_ERR_VALUE, "NULL data pointer");
     FM_REQUIRE(ldx >= in_rows && ldy >= out_rows && lda >= n, FM_ERR_VALUE,
                "leading dimension too small");
-    if (generic)
-        return dense_generic(a_dtype, adjoint, m, n, A, lda, x, ldx, y, ldy, k, as_stream(stream));
+    hipStream_t s = as_stream(stream);
+    switch (a_dtype) {
+    case FM_INT8: return gemm_generic<int8_t>(adjoint, m, n, A, lda, x, ldx, y, ldy, k, s);
+    case FM_INT16: return gemm_generic<int16_t>(adjoint, m, n, A, lda, x, ldx, y, ldy, k, s);
+    case FM_INT32: return gemm_generic<int32_t>(adjoint, m, n, A, lda, x, ldx, y, ldy, k, s);
+    case FM_INT64: return gemm_generic<int64_t>(adjoint, m, n, A, lda, x, ldx, y, ldy, k, s);
+    case FM_FLOAT64: return dense_direct<double, false>(adjoint, m, n, A, lda, x, ldx, y, ldy, k, s);
+    case FM_COMPLEX128:
+        return dense_direct<cpx<double>, false>(adjoint, m, n, A, lda, x, ldx, y, ldy, k, s);
+    default: break;
+    }
     GemmArgs g;
     memset(&g, 0, sizeof(g));
     g.M = out_rows;
@@ -479,7 +561,11 @@ extern "C" fm_status fm_dense_apply(int a_dtype, int x_dtype, int adjoint, int64
     g.bos = 0; g.brs = 1; g.bjs = ldx;
     g.Y = (float *)y;
     g.yos = 0; g.yrs = 1; g.yjs = ldy;
-    return gemm_launch(g, as_stream(stream));
+    // both sides at most 128: A stays in registers; larger ones load their
+    // operands as they go
+    if (gemm_is_small(g)) return gemm_launch_small(g, s);
+    if (g.cplx) return dense_direct<float, true>(adjoint, m, n, A, lda, x, ldx, y, ldy, k, s);
+    return dense_direct<float, false>(adjoint, m, n, A, lda, x, ldx, y, ldy, k, s);
 }
 
 extern "C" fm_status fm_dense_apply_strided(int a_dtype, int x_dtype, int adjoint, int64_t n,
@@ -505,5 +591,6 @@ extern "C" fm_status fm_dense_apply_strided(int a_dtype, int x_dtype, int adjoin
     g.bos = n * inner; g.brs = inner; g.bjs = 1;
     g.Y = (float *)y;
     g.yos = n * inner; g.yrs = inner; g.yjs = 1;
-    return gemm_launch(g, as_stream(stream));
+    return gemm_is_small(g) ? gemm_launch_small(g, as_stream(stream))
+                            : gemm_launch_tiled(g, as_stream(stream));
 }
