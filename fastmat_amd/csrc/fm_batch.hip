@@ -439,8 +439,7 @@ static fm_status finalize(ProgBuilder<T> &b, Program &prog, int ncu_lanes_cap, h
 template <typename T, int LOGN, bool CONV>
 static fm_status launch_pass_class(const fm_batch_plan *p, const Program &d, const Launch &l,
                                    hipStream_t s, int64_t out_shift, const T *out_mul) {
-    constexpr int N = 1 << LOGN;
-    const size_t lds = size_t(tile_batch<T>(LOGN)) * (N + (N >> 5) + 1) * sizeof(cpx<T>);
+    const size_t lds = tile_lds_bytes<T>(LOGN, tile_batch<T>(LOGN));
     static bool attr = false;
     if (!attr) {
         (void)hipFuncSetAttribute((const void *)batch_pass_kernel<T, LOGN, CONV, false>,
@@ -478,7 +477,7 @@ static fm_status launch_corr_nt(const fm_batch_plan *p, const Program &d, const 
     constexpr int N = 1 << LOGN;
     constexpr int LE = corr_loge<T>(LOGN);
     using S = TileShape<T, LOGN, NT, LE>;
-    const size_t lds = size_t(S::B) * (N + (N >> 5) + 1) * sizeof(cpx<T>);
+    const size_t lds = tile_lds_bytes<T>(LOGN, S::B);
     static bool attr = false;
     if (!attr) {
         (void)hipFuncSetAttribute((const void *)batch_corr_kernel<T, LOGN, NT, false>,

@@ -125,7 +125,7 @@ static fm_status launch_pass(const TileArgs<T> &a, hipStream_t stream) {
     constexpr int NT = PassCfg<T, LOGN>::NT;
     constexpr int LE = PassCfg<T, LOGN>::LE;
     constexpr int N = 1 << LOGN;
-    const size_t lds = size_t(a.B) * (N + (N >> 5) + 1) * sizeof(cpx<T>);
+    const size_t lds = tile_lds_bytes<T>(LOGN, a.B);
     static bool attr_set = false;
     if (!attr_set) {
         (void)hipFuncSetAttribute((const void *)fft_pass_kernel<T, LOGN, NT, CONV, false, LE>,

@@ -154,9 +154,31 @@ template <int LOGN, int LOGE, bool REV = false> struct FftPlan {
     }
 };
 
-// Padded LDS index: one spare slot every 32 elements keeps the strided
-// exchanges of the stages free of most bank conflicts.
-__device__ __forceinline__ int lpad(int n) { return n + (n >> 5); }
+// Padded LDS index: one spare slot every 32 elements (16 of 16 bytes) keeps
+// the strided exchanges of the stages free of most bank conflicts.
+template <typename T = float> __host__ __device__ __forceinline__ constexpr int lpad(int n) {
+    return n + (n >> (sizeof(T) == 4 ? 5 : 4));
+}
+
+// LDS elements between the sequences of a tile of 2^LOGB sequences of 2^LOGN.
+// Accesses in the sequence-fastest mapping take 32 lanes (16 of 16 bytes) at a
+// time, 2^LOGB sequences by 32 / 2^LOGB neighbouring elements (one slot apart
+// after padding), so rows 32 / 2^LOGB slots apart (modulo 32) put them into
+// distinct banks; with one spare slot the 1024-point strided tiles (8
+// sequences) hit each bank four times.  With TwiddleChain below, measured in
+// one step: the 1024-point column pass of 2^20 x 64 columns 353 -> 317 us (64 MB
+// of columns: 38.2 -> 34.6), Fourier 2^20 x 64 forward and adjoint 1058 ->
+// 1016 us, 50 FISTA iterations on 2^18 x 8 8256 -> 7748 us.
+template <typename T> __host__ __device__ constexpr int tile_row(int logn, int logb) {
+    const int span = sizeof(T) == 4 ? 32 : 16;
+    const int spare = logb == 0 ? 0 : ((span >> logb) > 1 ? (span >> logb) : 1);
+    return lpad<T>(1 << logn) + spare;
+}
+
+// LDS bytes of a tile of B (a power of two) sequences of 2^logn.
+template <typename T> inline size_t tile_lds_bytes(int logn, int B) {
+    return size_t(B) * tile_row<T>(logn, ilog2(B)) * sizeof(cpx<T>);
+}
 
 // ------------------------------------------------------------ tile kernel
 template <typename T> struct TileArgs {
@@ -328,6 +350,47 @@ __device__ __forceinline__ void bfly_pos(int g, bool seqfast, int &b, int &i) {
     }
 }
 
+// base * step^r for r = 0, 1, ... R - 1 in order, in FP64: up to four
+// interleaved recurrences by step^4, so that four products are in flight where
+// a single recurrence would wait for each (a product depends on the one four
+// back) and rounding errors pass through R / 4 products instead of R.
+template <int R> struct TwiddleChain {
+    static constexpr int C = R >= 8 ? 4 : (R >= 4 ? 2 : 1);
+    cpx<double> w[C], s;
+    // elements r = 0, 1, ...
+    __device__ __forceinline__ void start(cpx<double> base, cpx<double> step) {
+        start_powers(step);
+        if constexpr (C > 1) {
+#pragma unroll
+            for (int c = 1; c < C; ++c) w[c] = cmul(base, w[c]);
+        }
+        w[0] = base;
+    }
+    // the powers step^r alone, elements r = 1, 2, ...
+    __device__ __forceinline__ void start_powers(cpx<double> step) {
+        if constexpr (C == 1) {
+            s = step;
+        } else {
+            w[1] = step;
+            const cpx<double> s2 = cmul(step, step);
+            if constexpr (C == 2) {
+                s = s2;
+            } else {
+                w[2] = s2;
+                w[3] = cmul(step, s2);
+                s = cmul(s2, s2);
+            }
+        }
+        w[0] = s;
+    }
+    // element r, asked for in order
+    __device__ __forceinline__ cpx<double> at(int r) {
+        const cpx<double> t = w[r % C];
+        if (r + C < R) w[r % C] = cmul(t, s);
+        return t;
+    }
+};
+
 // One radix-2^LOGR stage with sub-length 2^LOGP on registers v (E per thread,
 // NB = E / R butterflies).  SRC: 0 = v already holds this stage's inputs,
 // 1 = read them from LDS.  DST: 0 = write outputs to LDS, 1 = leave them in v.
@@ -341,14 +404,14 @@ __device__ __forceinline__ void fft_stage2(cpx<T> *v, cpx<T> *lds,
     constexpr int R = 1 << LOGR, NB = E / R;
     constexpr int LOGNR = LOGN - LOGR, NR = 1 << LOGNR;
     constexpr int P = 1 << LOGP;
-    constexpr int SB = (1 << LOGN) + ((1 << LOGN) >> 5) + 1;
+    constexpr int SB = tile_row<T>(LOGN, LOGB);
     if constexpr (SRC == 1) {
 #pragma unroll
         for (int e = 0; e < NB; ++e) {
             int b, i;
             bfly_pos<LOGB, LOGNR>(threadIdx.x + e * NT, false, b, i);
 #pragma unroll
-            for (int r = 0; r < R; ++r) v[e * R + r] = lds[b * SB + lpad(i + r * NR)];
+            for (int r = 0; r < R; ++r) v[e * R + r] = lds[b * SB + lpad<T>(i + r * NR)];
         }
     }
 #pragma unroll
@@ -360,12 +423,12 @@ __device__ __forceinline__ void fft_stage2(cpx<T> *v, cpx<T> *lds,
             // W_{pR}^{r k} = W_N^{r k N / (p R)}: one FP64 lookup of
             // W_{pR}^k, its powers by FP64 products, rounded once to T
             const int step = k << (LOGN - LOGP - LOGR);
-            const cpx<double> w1 = ldg(tw, uint32_t(step));
-            cpx<double> w = w1;
+            TwiddleChain<R> w;
+            w.start_powers(ldg(tw, uint32_t(step)));
 #pragma unroll
             for (int r = 1; r < R; ++r) {
-                v[e * R + r] = twiddle_mul<SIGN>(v[e * R + r], mk(T(w.x), T(w.y)));
-                if (r + 1 < R) w = cmul(w, w1);
+                const cpx<double> t = w.at(r);
+                v[e * R + r] = twiddle_mul<SIGN>(v[e * R + r], mk(T(t.x), T(t.y)));
             }
         }
         dftr<LOGR, SIGN>(v + e * R);
@@ -379,7 +442,7 @@ __device__ __forceinline__ void fft_stage2(cpx<T> *v, cpx<T> *lds,
             const int k = i & (P - 1);
             const int base = ((i - k) << LOGR) + k;
 #pragma unroll
-            for (int r = 0; r < R; ++r) lds[b * SB + lpad(base + r * P)] = v[e * R + r];
+            for (int r = 0; r < R; ++r) lds[b * SB + lpad<T>(base + r * P)] = v[e * R + r];
         }
         __syncthreads();
     }
@@ -506,7 +569,7 @@ __device__ __forceinline__ void fft_tile_store(const TileArgs<T> &a, int64_t til
     constexpr int RL = 1 << LOGRL;
     constexpr int LOGB = S::LOGB;
     constexpr int B = S::B;
-    constexpr int SB = N + (N >> 5) + 1;
+    constexpr int SB = tile_row<T>(LOGN, LOGB);
     const int64_t s0 = tile_first_seq<T, LOGB>(a, tile);
     constexpr int NBL = E / RL;
     constexpr int LOGNRL = LOGN - LOGRL, NRL = 1 << LOGNRL;
@@ -518,7 +581,7 @@ __device__ __forceinline__ void fft_tile_store(const TileArgs<T> &a, int64_t til
             int b, i;
             bfly_pos<LOGB, LOGNRL>(threadIdx.x + e * NT, cur_sf, b, i);
 #pragma unroll
-            for (int r = 0; r < RL; ++r) lds[b * SB + lpad(i + r * NRL)] = v[e * RL + r];
+            for (int r = 0; r < RL; ++r) lds[b * SB + lpad<T>(i + r * NRL)] = v[e * RL + r];
         }
         __syncthreads();
 #pragma unroll
@@ -526,7 +589,7 @@ __device__ __forceinline__ void fft_tile_store(const TileArgs<T> &a, int64_t til
             int b, i;
             bfly_pos<LOGB, LOGNRL>(threadIdx.x + e * NT, want_sf, b, i);
 #pragma unroll
-            for (int r = 0; r < RL; ++r) v[e * RL + r] = lds[b * SB + lpad(i + r * NRL)];
+            for (int r = 0; r < RL; ++r) v[e * RL + r] = lds[b * SB + lpad<T>(i + r * NRL)];
         }
         cur_sf = want_sf;
     }
@@ -540,28 +603,25 @@ __device__ __forceinline__ void fft_tile_store(const TileArgs<T> &a, int64_t til
         bfly_pos<LOGB, LOGNRL>(threadIdx.x + e * NT, cur_sf, b, i);
         const SeqPos<Ix> sp = seq_pos<Ix>(a, s0 + b);
         if (!sp.ok) continue;
-        cpx<T> w[RL];
-        if (a.twb_hi || a.post) {
+        if (a.twb_hi) {
             // four-step twiddle W_L^{j n} for n = i + r NRL: the FP64 base
-            // W_L^{j i} times successive FP64 powers of W_L^{j NRL} (two
-            // table lookups each, j n < L), rounded once to T
-            cpx<double> tw = mk(1.0, 0.0), step = mk(1.0, 0.0);
-            if (a.twb_hi) {
-                const Ix e0 = sp.j * Ix(i), e1 = sp.j * Ix(NRL);
-                tw = cmul(ldg(a.twb_hi, Ix(e0 >> a.twb_shift)), ldg(a.twb_lo, Ix(e0 & lo_mask)));
-                step = cmul(ldg(a.twb_hi, Ix(e1 >> a.twb_shift)), ldg(a.twb_lo, Ix(e1 & lo_mask)));
-            }
+            // W_L^{j i} times FP64 powers of W_L^{j NRL} (two table lookups
+            // each, j n < L), rounded once to T
+            const Ix e0 = sp.j * Ix(i), e1 = sp.j * Ix(NRL);
+            TwiddleChain<RL> w;
+            w.start(cmul(ldg(a.twb_hi, Ix(e0 >> a.twb_shift)), ldg(a.twb_lo, Ix(e0 & lo_mask))),
+                    cmul(ldg(a.twb_hi, Ix(e1 >> a.twb_shift)), ldg(a.twb_lo, Ix(e1 & lo_mask))));
 #pragma unroll
             for (int r = 0; r < RL; ++r) {
-                const Ix n = Ix(i + r * NRL);
-                cpx<T> t = mk(T(1), T(0));
-                if (a.twb_hi) {
-                    t = mk(T(tw.x), T(a.twb_sign > 0 ? -tw.y : tw.y));
-                    if (r + 1 < RL) tw = cmul(tw, step);
-                }
-                const Ix gidx = n * out_gn + sp.j * out_gj;
-                if (a.post && gidx < mv) t = cmul(t, ldg(a.post, gidx));
-                w[r] = t;
+                const cpx<double> t = w.at(r);
+                v[e * RL + r] = cmul(v[e * RL + r], mk(T(t.x), T(a.twb_sign > 0 ? -t.y : t.y)));
+            }
+        }
+        if (a.post) {
+#pragma unroll
+            for (int r = 0; r < RL; ++r) {
+                const Ix gidx = Ix(i + r * NRL) * out_gn + sp.j * out_gj;
+                if (gidx < mv) v[e * RL + r] = cmul(v[e * RL + r], ldg(a.post, gidx));
             }
         }
 #pragma unroll
@@ -570,7 +630,6 @@ __device__ __forceinline__ void fft_tile_store(const TileArgs<T> &a, int64_t til
             const Ix gidx = n * out_gn + sp.j * out_gj;
             if (gidx >= mv) continue;
             cpx<T> u = v[e * RL + r];
-            if (a.twb_hi || a.post) u = cmul(u, w[r]);
             if (a.conj_out) u = conj(u);
             if (a.target) {
                 const cpx<T> d = u - ldg(a.target, Ix(sp.out_base + n * out_ns));
@@ -605,7 +664,7 @@ __device__ __forceinline__ void fft_tile_compute(const TileArgs<T> &a, int64_t t
     constexpr int R0 = 1 << LOGR0, RL = 1 << LOGRL;
     constexpr int LOGB = S::LOGB;
     constexpr int B = S::B;
-    constexpr int SB = N + (N >> 5) + 1;
+    constexpr int SB = tile_row<T>(LOGN, LOGB);
     const int64_t s0 = tile_first_seq<T, LOGB>(a, tile);
 
     // ---- conj, pre-multiply (zero-padded positions hold zeros already)

@@ -24,6 +24,8 @@
 // The factors act on different axes, so their order does not matter; the
 // adjoint of (Circulant x A) is the conjugate spectrum with A^T, which the
 // caller passes as the matrix (A is real).
+#include <algorithm>
+
 #include "fm_fft_plan.hpp"
 
 namespace fm {
@@ -205,10 +207,8 @@ extern "C" fm_status fm_kron_conv_dense_apply(const fm_conv_plan *plan, int conj
     t.stream_out = 3;
     k.y = (cpx<float> *)y;
     k.A = (const float *)M;
-    const size_t lds = size_t(KF_N) * (KF_N + (KF_N >> 5) + 1) * sizeof(cpx<float>) >
-                               size_t(KF_N) * KF_ROW * sizeof(cpx<float>)
-                           ? size_t(KF_N) * (KF_N + (KF_N >> 5) + 1) * sizeof(cpx<float>)
-                           : size_t(KF_N) * KF_ROW * sizeof(cpx<float>);
+    const size_t lds = std::max(tile_lds_bytes<float>(KF_LOGN, KF_N),
+                                size_t(KF_N) * KF_ROW * sizeof(cpx<float>));
     static bool attr = false;
     if (!attr) {
         (void)hipFuncSetAttribute((const void *)kron_conv_dense_kernel<true>,
