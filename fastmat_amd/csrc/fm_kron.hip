@@ -1,243 +1,252 @@
-// The last two factors of a Kron product, a 128-point Circulant and a dense
-// 128 x 128 float32 matrix, applied to complex64 data in one pass over HBM.
+// The last two factors of a Kron product, a Circulant of N = 64 or 128 points
+// and a dense M x M float32 matrix (M = 64, 96 or 128), applied to complex64
+// data in one pass over HBM.
 //
 // Replaces two mode passes of Kron._forward / _backward (Kron.pyx:267-303:
-// one factor per mode, each a full read and write of the data) for
-// x viewed as (outer, n = 128, m = 128) with the dense axis contiguous: for
-// every outer index the 128 x 128 slab (128 KB, contiguous in HBM) is read
-// once, transformed by both factors on the chip and written once.
+// one factor per mode, each a full read and write of the data) for x viewed as
+// (outer, n = N, m = M) with the dense axis contiguous: every N x M slab is
+// read, transformed by both factors on the chip and written once.  The factors
+// act on different axes, so their order does not matter; the adjoint of
+// (Circulant x A) is the conjugate spectrum with A^T, which the caller passes
+// as the matrix (A is real).
 //
-// Per slab, one 1024-thread workgroup:
-//   1. loads the slab into registers in the FFT tile layout (sequences along
-//      the contiguous axis, 128 of them, elements along the circulant axis);
-//   2. runs the circulant as forward FFT, spectrum, inverse FFT on the
-//      registers and LDS (the tile engine of fm_fft_core.hpp);
-//   3. writes the slab to LDS row-major (rows = circulant index, padded to
-//      132 complex so that the MFMA operand reads below hit 64 distinct
-//      banks) and multiplies it by the dense factor on FP32 MFMA: the 256
-//      real columns (circulant index, real / imaginary part) in two halves,
-//      16 waves as 8 row blocks of A (loaded into registers in the MFMA
-//      operand layout) x 2 halves, each half eight 16-column blocks, K = 128
-//      in 32 steps of v_mfma_f32_16x16x4f32;
-//   4. stages the result through LDS and stores it as contiguous 16-byte
-//      vectors.
-// The factors act on different axes, so their order does not matter; the
-// adjoint of (Circulant x A) is the conjugate spectrum with A^T, which the
-// caller passes as the matrix (A is real).
+// A workgroup of 4 N / 64 waves computes 64 of a slab's M output columns:
+//   1. Z[n][i] = sum_j A[i][j] X[n][j] on FP32 MFMA (v_mfma_f32_16x16x4f32),
+//      operands loaded straight into the MFMA layout: a wave owns 16 columns i
+//      (its rows of A stay in registers) and 64 of the rows n, real and
+//      imaginary parts as separate blocks; per step of 8 j a lane loads 16
+//      bytes of four rows, the next step's loads in flight during the MFMAs.
+//      Which row n an MFMA row stands for is free, and is chosen so that the
+//      16 rows in a lane's accumulators are n0 + r N / 16, r = 0 ... 15: the
+//      inputs of a radix-16 butterfly.
+//   2. The circulant along n, from those registers: radix 16 and N / 16, the
+//      spectrum, radix N / 16 and 16 back (Stockham stages as in
+//      fm_fft_core.hpp) with two exchanges through LDS.  From the first
+//      exchange on a wave's 64 lanes are 64 neighbouring columns i and share
+//      the butterfly, so twiddles and spectrum are wave-uniform.
+//   3. The last stage stores from registers, 512 contiguous bytes a wave.
+// LDS holds the 64 columns once (68 KB for N = 128), so two workgroups run per
+// CU and the MFMAs of one overlap the butterflies, exchanges and stores of the
+// other; the two workgroups of a slab are neighbours on one XCD, and the second
+// reads the slab from its L2.
+//
+// What bounds it: HBM 16 bytes and the MFMA pipes 2 M flop per complex element
+// (52 and 55 us for 2^24 elements at M = 128).
 #include <algorithm>
 
 #include "fm_fft_plan.hpp"
 
 namespace fm {
 
-typedef float kf_f32x4 __attribute__((ext_vector_type(4)));
-
-constexpr int KF_LOGN = 7;             // circulant length 128 (middle axis)
-constexpr int KF_N = 1 << KF_LOGN;
-constexpr int KF_M = 128;              // dense size (contiguous axis)
-constexpr int KF_NT = 1024;            // 16 wave64
-constexpr int KF_LE = 4;               // 16 elements per thread in the transform
-constexpr int KF_ROW = KF_M + 4;       // padded LDS row of the slab (complex)
-constexpr int KF_SLAB = KF_N * KF_M;   // elements per slab
+typedef float kp_f32x4 __attribute__((ext_vector_type(4)));
+typedef float kp_f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float kp_f32x4u __attribute__((ext_vector_type(4), aligned(8)));
 
 struct KronPairArgs {
-    TileArgs<float> t;  // the slab as FFT sequences (load side, twiddles, spectrum)
+    const cpx<float> *x;
     cpx<float> *y;
-    const float *A;     // the dense factor as applied, 128 x 128 row-major
+    const float *A;          // the dense factor as applied, M x M row-major
+    const cpx<float> *D;     // spectrum, N entries
+    const cpx<double> *tw;   // W_N^e
+    int conj_d;
 };
 
-template <bool I32>
-__global__ __launch_bounds__(KF_NT) void kron_conv_dense_kernel(const KronPairArgs k) {
-    using S = TileShape<float, KF_LOGN, KF_NT, KF_LE>;
-    using P = typename S::P;
-    using Ix = IdxT<I32>;
-    constexpr int E = S::E, LOGE = S::LOGE, LOGB = S::LOGB;
-    static_assert(S::B == KF_M, "one tile is one slab");
-    // radices of the forward transform's last stage and of the reversed inverse's
-    constexpr int LOGRF = P::bits(P::S - 1), RF = 1 << LOGRF, NBF = E / RF;
-    constexpr int LOGNRF = KF_LOGN - LOGRF, NRF = 1 << LOGNRF;
-    constexpr int LOGRL = P::bits(0), RL = 1 << LOGRL, NBL = E / RL;
-    constexpr int LOGNRL = KF_LOGN - LOGRL, NRL = 1 << LOGNRL;
+template <int LOGN, int M>
+__global__ __launch_bounds__(4 << LOGN, 4) void kron_pair_kernel(const KronPairArgs k) {
+    constexpr int N = 1 << LOGN, WN = N / 64, NT = 256 * WN;
+    constexpr int LOGB = 6, E = 16;
+    constexpr int SB = tile_row<float>(LOGN, LOGB);
+    constexpr int NR0 = N / 16;                       // radix-16 butterflies
+    constexpr int LOGR = LOGN - 4, R = 1 << LOGR;     // the other radix
+    constexpr int NB = E / R;                         // its butterflies per thread
+    constexpr int T = M / 8;                          // K steps
+    constexpr int IB = (M + 63) / 64;                 // workgroups per slab
+    static_assert(NT == (4 << LOGN) && M % 16 == 0, "shape");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cpx<float> *lds = reinterpret_cast<cpx<float> *>(smem_raw);
-    const float *ldsf = reinterpret_cast<const float *>(smem_raw);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const TileArgs<float> &t = k.t;
-    int64_t tile = blockIdx.x;
-    if (tile >= t.ntiles) return;  // uniform over the workgroup
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, h = lane >> 4;
+    const int wi = wave & 3, wn = wave >> 2;
+    const int64_t tile = xcd_remap(blockIdx.x, gridDim.x);
+    const int64_t slab = tile / IB;
+    const int i0 = int(tile - slab * IB) * 64;        // first column of the workgroup
+    const cpx<float> *x = k.x + slab * (int64_t(N) * M);
+    cpx<float> v[E];
 
-    for (; tile < t.ntiles; tile += gridDim.x) {
-        cpx<float> v[E];
-        fft_tile_load<float, KF_LOGN, KF_NT, I32, KF_LE>(t, tile, v);
-        // ---- circulant along the middle axis: forward, spectrum, inverse
-        bool sf = true;  // the load mapping: neighbouring lanes on neighbouring sequences
-        fft_all<float, KF_LOGN, LOGE, -1, KF_NT, LOGB, 0, 1>(v, lds, t.tw, sf);
-        if (P::S > 1) sf = false;
+    if (M % 64 == 0 || i0 + 16 * wi < M) {
+        // A[i][8 t + 2 h + s] of column i = i0 + 16 wi + r
+        float a[2 * T];
+        const uint32_t abase = uint32_t(i0 + 16 * wi + r) * M + 2 * h;
 #pragma unroll
-        for (int e = 0; e < NBF; ++e) {
-            int b, i;
-            bfly_pos<LOGB, LOGNRF>(tid + e * KF_NT, sf, b, i);
-#pragma unroll
-            for (int r = 0; r < RF; ++r) {
-                const cpx<float> d = t.D[i + r * NRF];
-                v[e * RF + r] = t.conj_d ? cmulc(v[e * RF + r], d) : cmul(v[e * RF + r], d);
-            }
+        for (int t = 0; t < T; ++t) {
+            const kp_f32x2u w = *reinterpret_cast<const kp_f32x2u *>(k.A + abase + 8 * t);
+            a[2 * t] = w.x;
+            a[2 * t + 1] = w.y;
         }
-        fft_all<float, KF_LOGN, LOGE, +1, KF_NT, LOGB, 0, 1, true>(v, lds, t.tw, sf);
-        if (P::S > 1) sf = false;
-        // ---- the slab to LDS, row n (circulant index), column b (dense input index)
-        __syncthreads();  // the transform's last LDS reads are done
+        // MFMA row m of block f is n = (m / 4 + 4 wn) + NR0 (4 f + m % 4)
+        const uint32_t xbase = uint32_t((r >> 2) + 4 * wn + NR0 * (r & 3)) * M + 2 * h;
+        kp_f32x4 re[4], im[4];
 #pragma unroll
-        for (int e = 0; e < NBL; ++e) {
-            int b, i;
-            bfly_pos<LOGB, LOGNRL>(tid + e * KF_NT, sf, b, i);
+        for (int f = 0; f < 4; ++f) re[f] = im[f] = kp_f32x4{0.f, 0.f, 0.f, 0.f};
+        kp_f32x4u cur[4], nxt[4];
+        auto load = [&](int t, kp_f32x4u *d) {
 #pragma unroll
-            for (int r = 0; r < RL; ++r) lds[(i + r * NRL) * KF_ROW + b] = v[e * RL + r];
-        }
-        // ---- dense factor along the contiguous axis on FP32 MFMA:
-        // D[i][c] = sum_j A[i][j] * slab[c >> 1][j].part(c & 1); wave w owns
-        // output rows 16 (w & 7) .. + 15 and the columns of half w >> 3
-        // (128 real columns: slab rows 64 (w >> 3) .. + 63), as eight 16 x 16
-        // blocks, K = 128 in 32 steps
-        const int rb = wave & 7, h = wave >> 3, q = lane & 15;
-        // this wave's rows of A in the MFMA operand layout, a[st] =
-        // A[16 rb + (lane & 15)][4 st + (lane >> 4)] (from L2: 64 KB shared by
-        // every workgroup)
-        float a[KF_M / 4];
-        {
-            // one base offset per lane, the k-steps at constant distances
-            const uint32_t base = (16 * rb + q) * KF_M + (lane >> 4);
+            for (int f = 0; f < 4; ++f)
+                d[f] = *reinterpret_cast<const kp_f32x4u *>(x + (xbase + 8 * t + 4 * f * NR0 * M));
+        };
+        load(0, cur);
 #pragma unroll
-            for (int st = 0; st < KF_M / 4; ++st) a[st] = ldg(k.A, uint32_t(base + 4 * st));
-        }
-        // every wave's slab rows are in LDS before any wave reads them (the
-        // A loads above are in flight meanwhile)
-        __syncthreads();
-        // column c = 128 h + 16 cb + q is row c >> 1 = 64 h + 8 cb + (q >> 1),
-        // part q & 1; with j = 4 st + (lane >> 4) every operand is this lane's
-        // base plus a constant
-        const float *bp =
-            ldsf + (((64 * h + (q >> 1)) * KF_ROW + (lane >> 4)) * 2 + (q & 1));
-        kf_f32x4 acc[8];
+        for (int t = 0; t < T; ++t) {
+            if (t + 1 < T) load(t + 1, nxt);
 #pragma unroll
-        for (int cb = 0; cb < 8; ++cb) acc[cb] = kf_f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int s = 0; s < 2; ++s)
 #pragma unroll
-        for (int st = 0; st < KF_M / 4; ++st) {
+                for (int f = 0; f < 4; ++f) {
+                    re[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur[f][2 * s], a[2 * t + s],
+                                                                 re[f], 0, 0, 0);
+                    im[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur[f][2 * s + 1], a[2 * t + s],
+                                                                 im[f], 0, 0, 0);
+                }
 #pragma unroll
-            for (int cb = 0; cb < 8; ++cb) {
-                const float bv = bp[(8 * cb * KF_ROW + 4 * st) * 2];
-                acc[cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[st], bv, acc[cb], 0, 0, 0);
-            }
-            // keep the scheduler from hoisting every k-step's operand reads
-            // (the unrolled loop would hold them all in registers; grouping
-            // 2 or 4 k-steps per barrier spilled and measured 9% slower)
+            for (int f = 0; f < 4; ++f) cur[f] = nxt[f];
+            // one step's loads in flight, not all of them hoisted into registers
             __builtin_amdgcn_sched_barrier(0);
         }
-        __syncthreads();  // every wave is done reading the slab
-        // ---- stage the result: D[i][c], i = 16 rb + 4 (lane >> 4) + u, goes
-        // to row c >> 1, column i
-        {
-            float *wp = reinterpret_cast<float *>(smem_raw) +
-                        (((64 * h + (q >> 1)) * KF_ROW + 16 * rb + 4 * (lane >> 4)) * 2 + (q & 1));
 #pragma unroll
-            for (int cb = 0; cb < 8; ++cb)
+        for (int f = 0; f < 4; ++f)
 #pragma unroll
-                for (int u = 0; u < 4; ++u) wp[(8 * cb * KF_ROW + u) * 2] = acc[cb][u];
-        }
-        __syncthreads();
-        {
-            const Ix base = Ix(tile) * Ix(KF_SLAB);
-            constexpr int PER = KF_SLAB / 2 / KF_NT;  // pairs of elements per thread
+            for (int u = 0; u < 4; ++u) v[4 * f + u] = mk(re[f][u], im[f][u]);
+        // radix 16 of butterfly n0 = h + 4 wn, column 16 wi + r
+        dftr<4, -1>(v);
+        const int base = (16 * wi + r) * SB, n0 = h + 4 * wn;
 #pragma unroll
-            for (int e = 0; e < PER; ++e) {
-                const int p = tid + e * KF_NT;        // pair index in the slab
-                const int n = (2 * p) / KF_M, i = (2 * p) % KF_M;
-                const float4 w = *reinterpret_cast<const float4 *>(&lds[n * KF_ROW + i]);
-                if (t.stream_out & 1) {
-                    FM_GLOBAL kf_f32x4 *q = (FM_GLOBAL kf_f32x4 *)(FM_GLOBAL char *)k.y +
-                                            (base / 2 + Ix(p));
-                    __builtin_nontemporal_store(kf_f32x4{w.x, w.y, w.z, w.w}, q);
-                } else {
-                    stg(reinterpret_cast<float4 *>(k.y), Ix(base / 2 + Ix(p)), w);
-                }
-            }
-        }
-        __syncthreads();  // the LDS is rewritten by the next slab's transform
+        for (int q = 0; q < 16; ++q) lds[base + lpad(16 * n0 + q)] = v[q];
     }
+    __syncthreads();
+
+    // from here lane = column, butterflies i = wave + e NT / 64 (wave-uniform)
+    const int row = lane * SB;
+#pragma unroll
+    for (int e = 0; e < NB; ++e) {
+        const int i = wave + e * (NT / 64);           // < 16
+        cpx<float> *w = v + e * R;
+#pragma unroll
+        for (int q = 0; q < R; ++q) w[q] = lds[row + lpad(i + 16 * q)];
+        TwiddleChain<R> c;
+        c.start_powers(k.tw[i]);
+#pragma unroll
+        for (int q = 1; q < R; ++q) {
+            const cpx<double> t = c.at(q);
+            w[q] = cmul(w[q], mk(float(t.x), float(t.y)));
+        }
+        dftr<LOGR, -1>(w);
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const cpx<float> d = k.D[i + 16 * q];
+            w[q] = k.conj_d ? cmulc(w[q], d) : cmul(w[q], d);
+        }
+        dftr<LOGR, +1>(w);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < NB; ++e) {
+        const int i = wave + e * (NT / 64);
+#pragma unroll
+        for (int q = 0; q < R; ++q) lds[row + lpad(R * i + q)] = v[e * R + q];
+    }
+    __syncthreads();
+    {
+        const int i = wave;                           // < NR0 = R
+#pragma unroll
+        for (int q = 0; q < 16; ++q) v[q] = lds[row + lpad(i + NR0 * q)];
+        TwiddleChain<16> c;
+        c.start_powers(k.tw[i]);
+#pragma unroll
+        for (int q = 1; q < 16; ++q) {
+            const cpx<double> t = c.at(q);
+            v[q] = cmulc(v[q], mk(float(t.x), float(t.y)));
+        }
+        dftr<4, +1>(v);
+        if (M % 64 != 0 && i0 + lane >= M) return;
+        cpx<float> *y = k.y + slab * (int64_t(N) * M) + i0;
+#pragma unroll
+        for (int q = 0; q < 16; ++q)
+            stg_stream(y, uint32_t((i + NR0 * q) * M + lane), v[q]);
+    }
+}
+
+template <int LOGN, int M>
+static fm_status kron_pair_launch(const KronPairArgs &k, int64_t outer, hipStream_t stream) {
+    constexpr int N = 1 << LOGN;
+    const size_t lds = tile_lds_bytes<float>(LOGN, 64);
+    static bool attr = false;
+    if (!attr) {
+        (void)hipFuncSetAttribute((const void *)kron_pair_kernel<LOGN, M>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        attr = true;
+    }
+    const int64_t grid = outer * ((M + 63) / 64);
+    FM_REQUIRE(grid < (int64_t(1) << 31), FM_ERR_VALUE, "too many slabs for one launch");
+    ProfToken tok;
+    prof_begin(stream, &tok);
+    hipLaunchKernelGGL((kron_pair_kernel<LOGN, M>), dim3(unsigned(grid)), dim3(4 << LOGN), lds,
+                       stream, k);
+    FM_CHECK_LAUNCH();
+    if (tok.active) {
+        const double bytes = 2.0 * double(outer) * N * M * 8.0 + double(M) * M * 4.0 + N * 8.0;
+        prof_end(stream, &tok, "kron_pair_kernel", bytes,
+                 4.0 * double(M) * M * double(N) * double(outer));
+    }
+    return FM_SUCCESS;
 }
 
 }  // namespace fm
 
 using namespace fm;
 
-extern "C" fm_status fm_kron_conv_dense_apply(const fm_conv_plan *plan, int conj_circulant,
-                                              const void *M, int64_t ldm, const void *x, void *y,
-                                              int64_t outer, void *stream) {
-    FM_REQUIRE(plan != nullptr && M != nullptr, FM_ERR_VALUE, "NULL plan or matrix");
-    FM_REQUIRE(plan->kind != 2 && plan->prec == FM_COMPLEX64 && plan->rows == KF_N &&
-                   plan->cols == KF_N && plan->L == KF_N,
+extern "C" fm_status fm_kron_pair_apply(const fm_conv_plan *plan, int conj_circulant,
+                                        const void *A, int64_t m, const void *x, void *y,
+                                        int64_t outer, void *stream) {
+    FM_REQUIRE(plan != nullptr && A != nullptr, FM_ERR_VALUE, "NULL plan or matrix");
+    const int64_t n = plan->rows;
+    FM_REQUIRE(plan->kind != 2 && plan->prec == FM_COMPLEX64 && plan->cols == n && plan->L == n &&
+                   (n == 64 || n == 128) && (m == 64 || m == 96 || m == 128),
                FM_ERR_NOT_IMPLEMENTED,
-               "the fused Kron pair needs a complex64 128-point Circulant plan");
-    FM_REQUIRE(ldm == KF_M, FM_ERR_VALUE, "the fused Kron pair needs a contiguous 128 x 128 matrix");
+               "the fused Kron pair needs a complex64 Circulant plan of 64 or 128 points and a "
+               "matrix of 64, 96 or 128 rows");
     FM_REQUIRE(outer >= 0, FM_ERR_VALUE, "negative slab count");
     if (outer == 0) return FM_SUCCESS;
     FM_REQUIRE(x != nullptr && y != nullptr, FM_ERR_VALUE, "NULL data pointer");
     FM_REQUIRE(x != y, FM_ERR_VALUE, "the fused Kron pair does not run in place");
-    FM_REQUIRE((uintptr_t(y) & 15) == 0, FM_ERR_VALUE, "output must be 16-byte aligned");
     KronPairArgs k;
-    memset(&k, 0, sizeof(k));
-    TileArgs<float> &t = k.t;
-    t = blank_args<float>();
-    t.logN = KF_LOGN;
-    t.O = outer;
-    t.J = KF_M;
-    t.B = KF_M;
-    t.ntiles = outer;
-    t.logJ = 7;
-    t.x = (const cpx<float> *)x;
-    t.in_os = KF_SLAB; t.in_js = 1; t.in_ns = KF_M;
-    t.in_gn = 1; t.in_gj = 0;
-    t.seqfast_in = 1;
-    t.tw = (const cpx<double> *)plan->geo.tw_full;
-    t.D = (const cpx<float> *)plan->D;
-    t.d_gn = 1; t.d_gj = 0;
-    t.conj_d = conj_circulant ? 1 : 0;
-    // the slabs are read once and written once: non-temporal loads and
-    // stores (the kron workload 0.53 -> 0.50 ms per step)
-    t.stream_out = 3;
+    k.x = (const cpx<float> *)x;
     k.y = (cpx<float> *)y;
-    k.A = (const float *)M;
-    const size_t lds = std::max(tile_lds_bytes<float>(KF_LOGN, KF_N),
-                                size_t(KF_N) * KF_ROW * sizeof(cpx<float>));
-    static bool attr = false;
-    if (!attr) {
-        (void)hipFuncSetAttribute((const void *)kron_conv_dense_kernel<true>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        (void)hipFuncSetAttribute((const void *)kron_conv_dense_kernel<false>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        attr = true;
-    }
-    int dev = 0, ncu = 256;
-    if (hipGetDevice(&dev) == hipSuccess)
-        (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    int64_t grid = ncu;
-    if (grid > outer) grid = outer;
-    // 32-bit element offsets when the whole block stays below 4 GiB
-    const bool i32 = double(outer) * KF_SLAB * sizeof(cpx<float>) < 4294967296.0;
-    ProfToken tok;
-    prof_begin(as_stream(stream), &tok);
-    const dim3 gd = dim3(unsigned(grid)), bd = dim3(KF_NT);
+    k.A = (const float *)A;
+    k.D = (const cpx<float> *)plan->D;
+    k.tw = (const cpx<double> *)plan->geo.tw_full;
+    k.conj_d = conj_circulant ? 1 : 0;
     hipStream_t s = as_stream(stream);
-    if (i32)
-        hipLaunchKernelGGL((kron_conv_dense_kernel<true>), gd, bd, lds, s, k);
-    else
-        hipLaunchKernelGGL((kron_conv_dense_kernel<false>), gd, bd, lds, s, k);
-    FM_CHECK_LAUNCH();
-    if (tok.active) {
-        const double bytes = 2.0 * double(outer) * KF_SLAB * sizeof(cpx<float>) +
-                             double(KF_M) * KF_M * 4.0 + double(KF_N) * 8.0;
-        const double flops = 2.0 * double(KF_M) * KF_M * 2.0 * double(KF_N) * double(outer);
-        prof_end(as_stream(stream), &tok, "kron_conv_dense_kernel", bytes, flops);
-    }
-    return FM_SUCCESS;
+    if (n == 64)
+        return m == 64   ? kron_pair_launch<6, 64>(k, outer, s)
+               : m == 96 ? kron_pair_launch<6, 96>(k, outer, s)
+                         : kron_pair_launch<6, 128>(k, outer, s);
+    return m == 64   ? kron_pair_launch<7, 64>(k, outer, s)
+           : m == 96 ? kron_pair_launch<7, 96>(k, outer, s)
+                     : kron_pair_launch<7, 128>(k, outer, s);
+}
+
+extern "C" fm_status fm_kron_conv_dense_apply(const fm_conv_plan *plan, int conj_circulant,
+                                              const void *M, int64_t ldm, const void *x, void *y,
+                                              int64_t outer, void *stream) {
+    FM_REQUIRE(plan != nullptr && M != nullptr, FM_ERR_VALUE, "NULL plan or matrix");
+    FM_REQUIRE(plan->kind != 2 && plan->prec == FM_COMPLEX64 && plan->rows == 128 &&
+                   plan->cols == 128 && plan->L == 128,
+               FM_ERR_NOT_IMPLEMENTED,
+               "the fused Kron pair needs a complex64 128-point Circulant plan");
+    FM_REQUIRE(ldm == 128, FM_ERR_VALUE, "the fused Kron pair needs a contiguous 128 x 128 matrix");
+    FM_REQUIRE(outer >= 0, FM_ERR_VALUE, "negative slab count");
+    FM_REQUIRE(outer == 0 || (uintptr_t(y) & 15) == 0, FM_ERR_VALUE,
+               "output must be 16-byte aligned");
+    return fm_kron_pair_apply(plan, conj_circulant, M, ldm, x, y, outer, stream);
 }

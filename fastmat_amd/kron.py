@@ -68,14 +68,14 @@ class Kron(Matrix):
             inner = int(np.prod(dims[m + 1:], dtype=np.int64))
             X = _apply_mode(f, X, adjoint, outer, dims[m], inner)
         if fused:
-            # the last two factors (Circulant(128), dense 128 x 128 float32)
-            # in one pass over the data (fm_kron_conv_dense_apply)
+            # the last two factors (a Circulant and a dense float32 matrix)
+            # in one pass over the data (fm_kron_pair_apply)
             C, A = self._content[-2:]
             Xc = X.contiguous()
             Y = torch.empty_like(Xc)
             outer = k * int(np.prod(dims[:-2], dtype=np.int64))
-            _lib.call("fm_kron_conv_dense_apply", C.plan_handle(np.complex64), int(adjoint),
-                      _lib.ptr(A._device_f32(transposed=adjoint)), 128, _lib.ptr(Xc),
+            _lib.call("fm_kron_pair_apply", C.plan_handle(np.complex64), int(adjoint),
+                      _lib.ptr(A._device_f32(transposed=adjoint)), A.numRows, _lib.ptr(Xc),
                       _lib.ptr(Y), outer, D.stream())
             X = Y
         return X
@@ -94,16 +94,16 @@ class Kron(Matrix):
 
 
 def _fused_tail(content, dtype):
-    """True when the product ends in a one-level Circulant of 128 points and a
-    dense 128 x 128 float32 Matrix and the data is complex64: those two modes
-    then run as one pass (the fused kernel's only shape)."""
+    """True when the product ends in a one-level Circulant of 64 or 128 points
+    and a dense float32 Matrix of 64, 96 or 128 rows and the data is complex64:
+    those two modes then run as one pass (the fused kernel's shapes)."""
     from .circulant import Circulant
     if len(content) < 2 or D.np_dtype(dtype) != np.dtype(np.complex64):
         return False
     C, A = content[-2:]
-    return (type(C) is Circulant and C._multi is None and C.numRows == 128 and
+    return (type(C) is Circulant and C._multi is None and C.numRows in (64, 128) and
             C.compute_dtype(dtype) == np.dtype(np.complex64) and
-            type(A) is Matrix and A.numRows == 128 and A.numCols == 128 and
+            type(A) is Matrix and A.numRows in (64, 96, 128) and A.numCols == A.numRows and
             A._array.dtype == np.float32)
 
 
