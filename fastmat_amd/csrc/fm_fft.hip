@@ -233,6 +233,9 @@ fm_status make_geometry(int prec, int logL, bool conv, hipStream_t stream, Geome
     if ((int64_t(1) << logL) <= single_max) {
         g->passes = 1;
         g->tw_full = twiddle_table(FM_COMPLEX128, logL, stream, &st);
+        // the fused Kron pair reads its twiddles as they are (fm_kron.hip)
+        if (!st && prec == FM_COMPLEX64 && (logL == 6 || logL == 7))
+            g->tw32 = twiddle_table(FM_COMPLEX64, logL, stream, &st);
         return st;
     }
     g->logN1 = logL / 2;

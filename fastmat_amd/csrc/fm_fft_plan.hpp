@@ -97,6 +97,7 @@ struct Geometry {
     int logN1, logN2;
     const void *tw_full, *tw1, *tw2, *twb_hi, *twb_lo;
     int twb_shift;
+    const void *tw32;  // complex64 plans of 64 and 128 points: W_L^e rounded to FP32
 };
 
 fm_status make_geometry(int prec, int logL, bool conv, hipStream_t stream, Geometry *g);
