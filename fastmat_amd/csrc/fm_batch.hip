@@ -66,10 +66,11 @@ template <typename T> struct CorrDesc {
     int mode;            // CorrMode
 };
 
-// One persistent kernel per (length, conv) class: grid-strided over the
-// class's (descriptor, tile) items.
-template <typename T, int LOGN, bool CONV, bool I32>
-__global__ __launch_bounds__((PassCfg<T, LOGN>::NT)) void batch_pass_kernel(
+// One persistent kernel per (length, conv, shape) class: grid-strided over the
+// class's (descriptor, tile) items.  SHAPE is SHAPE_WIDE or SHAPE_ROW (a batch
+// has no small launches).
+template <typename T, int LOGN, bool CONV, int SHAPE, bool I32>
+__global__ __launch_bounds__((PassCfg<T, LOGN, SHAPE>::NT)) void batch_pass_kernel(
     const BatchDesc<T> *__restrict__ descs, const int2 *__restrict__ items, int64_t nitems,
     int64_t out_shift, const T *__restrict__ out_mul) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -83,7 +84,8 @@ __global__ __launch_bounds__((PassCfg<T, LOGN>::NT)) void batch_pass_kernel(
             a.y = reinterpret_cast<cpx<T> *>(reinterpret_cast<char *>(a.y) + out_shift);
             if (out_mul) a.out_scale *= *out_mul;
         }
-        fft_pass_body<T, LOGN, PassCfg<T, LOGN>::NT, CONV, I32, PassCfg<T, LOGN>::LE>(a, w.y, lds);
+        fft_pass_body<T, LOGN, PassCfg<T, LOGN, SHAPE>::NT, CONV, I32,
+                      PassCfg<T, LOGN, SHAPE>::LE>(a, w.y, lds);
         __syncthreads();  // the next item reuses the LDS tile
     }
 }
@@ -195,7 +197,7 @@ enum LaunchKind { LK_FFT = 0, LK_CONV = 1, LK_CORR = 2 };
 
 // One launch of a program: the work items of one kernel class on one lane.
 struct Launch {
-    int kind, logN, nt, lane;
+    int kind, logN, nt, lane;  // nt: threads of a correlation, shape of a pass
     int early;  // from a pass group that needs no spectrum
     int idx32;  // every descriptor of the launch fits 32-bit index arithmetic
     void *items;
@@ -322,12 +324,19 @@ static double pass_bytes(const TileArgs<double> &a, size_t esz) {
     return (in + out) * double(esz);
 }
 
+// Tiling of a batch pass (its class's shape, see batch_pass_kernel).
+template <typename T> static fm_status normalize_batch_pass(TileArgs<T> &a) {
+    FM_REQUIRE(a.logN >= 0 && a.logN <= batch_max_log<T>(), FM_ERR_VALUE,
+               "batched transform length 2^%d out of range", a.logN);
+    return normalize_pass(a, pass_batch<T>(a.logN, pick_shape(a, false)));
+}
+
 // Normalise the descriptors, group work items into launches and upload.
 template <typename T>
 static fm_status finalize(ProgBuilder<T> &b, Program &prog, int ncu_lanes_cap, hipStream_t s) {
     free_program(prog);
     for (auto &d : b.descs) {
-        fm_status st = normalize_pass(d.a);
+        fm_status st = normalize_batch_pass(d.a);
         if (st) return st;
         // the batch's passes write gigabytes per launch that the next pass
         // reads back long after: non-temporal stores and loads (the
@@ -375,7 +384,8 @@ static fm_status finalize(ProgBuilder<T> &b, Program &prog, int ncu_lanes_cap, h
         for (const auto &r : pg.refs) {
             const TileArgs<T> &a = r.corr ? b.cdescs[r.index].a : b.descs[r.index].a;
             int kind = r.corr ? LK_CORR : (b.descs[r.index].conv ? LK_CONV : LK_FFT);
-            int nt = r.corr ? corr_threads(a.logN, corr_loge<T>(a.logN), a.J > 1) : 0;
+            int nt = r.corr ? corr_threads(a.logN, corr_loge<T>(a.logN), a.J > 1)
+                            : pick_shape(a, false);
             auto key = std::make_tuple(kind, a.logN, nt);
             bool fit = fits_idx32(a, int64_t(1) << a.logN);
             if (r.corr) {
@@ -436,15 +446,15 @@ static fm_status finalize(ProgBuilder<T> &b, Program &prog, int ncu_lanes_cap, h
 }
 
 // ------------------------------------------------------------- launching
-template <typename T, int LOGN, bool CONV>
-static fm_status launch_pass_class(const fm_batch_plan *p, const Program &d, const Launch &l,
+template <typename T, int LOGN, bool CONV, int SHAPE>
+static fm_status launch_pass_shape(const fm_batch_plan *p, const Program &d, const Launch &l,
                                    hipStream_t s, int64_t out_shift, const T *out_mul) {
-    const size_t lds = tile_lds_bytes<T>(LOGN, tile_batch<T>(LOGN));
+    const size_t lds = tile_lds_bytes<T>(LOGN, pass_batch<T>(LOGN, SHAPE));
     static bool attr = false;
     if (!attr) {
-        (void)hipFuncSetAttribute((const void *)batch_pass_kernel<T, LOGN, CONV, false>,
+        (void)hipFuncSetAttribute((const void *)batch_pass_kernel<T, LOGN, CONV, SHAPE, false>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        (void)hipFuncSetAttribute((const void *)batch_pass_kernel<T, LOGN, CONV, true>,
+        (void)hipFuncSetAttribute((const void *)batch_pass_kernel<T, LOGN, CONV, SHAPE, true>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         attr = true;
     }
@@ -452,13 +462,13 @@ static fm_status launch_pass_class(const fm_batch_plan *p, const Program &d, con
     if (grid > l.nitems) grid = l.nitems;
     ProfToken tok;
     prof_begin(s, &tok);
-    constexpr int NT = PassCfg<T, LOGN>::NT;
+    constexpr int NT = PassCfg<T, LOGN, SHAPE>::NT;
     if (l.idx32)
-        hipLaunchKernelGGL((batch_pass_kernel<T, LOGN, CONV, true>), dim3(unsigned(grid)), dim3(NT),
-                           lds, s, (const BatchDesc<T> *)d.descs, (const int2 *)l.items, l.nitems,
-                           out_shift, out_mul);
+        hipLaunchKernelGGL((batch_pass_kernel<T, LOGN, CONV, SHAPE, true>), dim3(unsigned(grid)),
+                           dim3(NT), lds, s, (const BatchDesc<T> *)d.descs, (const int2 *)l.items,
+                           l.nitems, out_shift, out_mul);
     else
-        hipLaunchKernelGGL((batch_pass_kernel<T, LOGN, CONV, false>), dim3(unsigned(grid)),
+        hipLaunchKernelGGL((batch_pass_kernel<T, LOGN, CONV, SHAPE, false>), dim3(unsigned(grid)),
                            dim3(NT), lds, s, (const BatchDesc<T> *)d.descs, (const int2 *)l.items,
                            l.nitems, out_shift, out_mul);
     FM_CHECK_LAUNCH();
@@ -469,6 +479,14 @@ static fm_status launch_pass_class(const fm_batch_plan *p, const Program &d, con
         prof_end(s, &tok, name, l.bytes, 0.0, l.pass_bytes);
     }
     return FM_SUCCESS;
+}
+
+template <typename T, int LOGN, bool CONV>
+static fm_status launch_pass_class(const fm_batch_plan *p, const Program &d, const Launch &l,
+                                   hipStream_t s, int64_t out_shift, const T *out_mul) {
+    if (l.nt == SHAPE_ROW)
+        return launch_pass_shape<T, LOGN, CONV, SHAPE_ROW>(p, d, l, s, out_shift, out_mul);
+    return launch_pass_shape<T, LOGN, CONV, SHAPE_WIDE>(p, d, l, s, out_shift, out_mul);
 }
 
 template <typename T, int LOGN, int NT>
@@ -816,7 +834,7 @@ static fm_status batch_bind_t(fm_batch_plan *p, int adjoint, const void *const *
             FM_REQUIRE(targets[i] != nullptr && ld_t[i] == ld_out[i], FM_ERR_VALUE,
                        "batch entry %d: target missing or with another leading dimension", i);
             TileArgs<T> a = pipes[i].back().a;
-            fm_status st = normalize_pass(a);
+            fm_status st = normalize_batch_pass(a);
             if (st) return st;
             slots += a.ntiles;
         }
@@ -831,7 +849,7 @@ static fm_status batch_bind_t(fm_batch_plan *p, int adjoint, const void *const *
             a.res_base = base;
             a.out_scale = T(res_scale);
             TileArgs<T> n = a;
-            (void)normalize_pass(n);
+            (void)normalize_batch_pass(n);
             base += n.ntiles;
         }
         p->n_res = slots;
@@ -967,7 +985,7 @@ static fm_status batch_bind_lsq_t(fm_batch_plan *p, const void *const *ins, cons
     std::vector<int64_t> base(p->count);
     for (int i = 0; i < p->count; ++i) {
         TileArgs<T> a = fw[i].back().a;
-        fm_status st = normalize_pass(a);
+        fm_status st = normalize_batch_pass(a);
         if (st) return st;
         base[i] = slots;
         slots += a.ntiles;

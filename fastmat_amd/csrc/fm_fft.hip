@@ -120,99 +120,6 @@ const void *twiddle_table(int precision, int logn, hipStream_t stream, fm_status
     return table(precision, logn, int64_t(1) << logn, stream, st);
 }
 
-template <typename T, int LOGN, bool CONV>
-static fm_status launch_pass(const TileArgs<T> &a, hipStream_t stream) {
-    constexpr int NT = PassCfg<T, LOGN>::NT;
-    constexpr int LE = PassCfg<T, LOGN>::LE;
-    constexpr int N = 1 << LOGN;
-    const size_t lds = tile_lds_bytes<T>(LOGN, a.B);
-    static bool attr_set = false;
-    if (!attr_set) {
-        (void)hipFuncSetAttribute((const void *)fft_pass_kernel<T, LOGN, NT, CONV, false, LE>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        (void)hipFuncSetAttribute((const void *)fft_pass_kernel<T, LOGN, NT, CONV, true, LE>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        attr_set = true;
-    }
-    FM_REQUIRE(lds <= 160 * 1024, FM_ERR_VALUE, "tile of %d x %d needs %zu bytes of LDS", a.B, N,
-               lds);
-    FM_REQUIRE(a.ntiles > 0 && a.ntiles < (int64_t(1) << 31), FM_ERR_VALUE,
-               "tile count %lld out of range", (long long)a.ntiles);
-    const bool i32 = fits_idx32(a, N);
-    // 1024-point complex64 passes that also multiply by a chirp (Bluestein
-    // pass A / C) run the 16-element, 512-thread shape: with the chirp loads
-    // they gain more from the extra waves than they lose to the extra stage
-    // (plain 1024-point passes are faster with 32 elements per thread)
-    bool e16 = false;
-    if constexpr (sizeof(T) == 4 && LOGN == 10) e16 = i32 && (a.pre || a.post);
-    ProfToken tok;
-    prof_begin(stream, &tok);
-    if constexpr (sizeof(T) == 4 && LOGN == 10) {
-        if (e16) {
-            static bool attr16 = false;
-            if (!attr16) {
-                (void)hipFuncSetAttribute((const void *)fft_pass_kernel<T, LOGN, 512, CONV, true, 4>,
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-                attr16 = true;
-            }
-            hipLaunchKernelGGL((fft_pass_kernel<T, LOGN, 512, CONV, true, 4>),
-                               dim3(unsigned(a.ntiles)), dim3(512), lds, stream, a);
-        }
-    }
-    if (!e16) {
-        if (i32)
-            hipLaunchKernelGGL((fft_pass_kernel<T, LOGN, NT, CONV, true, LE>),
-                               dim3(unsigned(a.ntiles)), dim3(NT), lds, stream, a);
-        else
-            hipLaunchKernelGGL((fft_pass_kernel<T, LOGN, NT, CONV, false, LE>),
-                               dim3(unsigned(a.ntiles)), dim3(NT), lds, stream, a);
-    }
-    FM_CHECK_LAUNCH();
-    if (tok.active) {
-        const double span = double(a.J) * N;
-        const double esz = double(sizeof(cpx<T>));
-        const double in = double(a.O) * (double(a.n_valid) < span ? double(a.n_valid) : span);
-        const double out = double(a.O) * (double(a.m_valid) < span ? double(a.m_valid) : span);
-        const double spec = CONV ? (a.d_gj ? span : double(N)) : 0.0;
-        char name[96];
-        snprintf(name, sizeof(name), "fft_pass_kernel<%s,%d,%d,%s>",
-                 sizeof(T) == 4 ? "float" : "double", LOGN, e16 ? 512 : NT,
-                 CONV ? "conv" : "fft");
-        const double nseq = double(a.O) * double(a.J);
-        const double flops = nseq * 5.0 * N * LOGN * (CONV ? 2.0 : 1.0);
-        const double own = (in + out + spec) * esz;
-        prof_end(stream, &tok, name, a.alg_bytes > 0 ? a.alg_bytes : own, flops, own);
-    }
-    return FM_SUCCESS;
-}
-
-template <typename T>
-fm_status launch_tile(const TileArgs<T> &a_in, bool conv, hipStream_t stream) {
-    TileArgs<T> a = a_in;
-    fm_status nst = normalize_pass(a);
-    if (nst) return nst;
-#define FM_PASS_CASE(L)                                                                  \
-    case L:                                                                              \
-        return conv ? launch_pass<T, L, true>(a, stream) : launch_pass<T, L, false>(a, stream);
-    switch (a.logN) {
-        FM_PASS_CASE(0) FM_PASS_CASE(1) FM_PASS_CASE(2) FM_PASS_CASE(3) FM_PASS_CASE(4)
-        FM_PASS_CASE(5) FM_PASS_CASE(6) FM_PASS_CASE(7) FM_PASS_CASE(8) FM_PASS_CASE(9)
-        FM_PASS_CASE(10) FM_PASS_CASE(11) FM_PASS_CASE(12) FM_PASS_CASE(13)
-    case 14:
-        if constexpr (sizeof(T) == 4)
-            return conv ? launch_pass<T, 14, true>(a, stream) : launch_pass<T, 14, false>(a, stream);
-        break;
-    default:
-        break;
-    }
-#undef FM_PASS_CASE
-    set_error("unsupported sub-transform length 2^%d", a.logN);
-    return FM_ERR_VALUE;
-}
-
-template fm_status launch_tile<float>(const TileArgs<float> &, bool, hipStream_t);
-template fm_status launch_tile<double>(const TileArgs<double> &, bool, hipStream_t);
-
 // Tile-shape knob: environment override (used by the tuning sweeps), else
 // the built-in default.
 int knob(const char *name, int dflt) {

@@ -786,38 +786,97 @@ __global__ __launch_bounds__(NT) void fft_pass_kernel(const TileArgs<T> a) {
                                               reinterpret_cast<cpx<T> *>(smem_raw));
 }
 
-// Host-side launcher for one tile pass (defined in fm_fft.hip).
+// Host-side launcher for one pass: plain or spectrum (defined in
+// fm_fft_pass_*.hip).
+template <typename T, bool CONV>
+fm_status launch_kind(const TileArgs<T> &a, hipStream_t stream);
 template <typename T>
-fm_status launch_tile(const TileArgs<T> &a, bool conv, hipStream_t stream);
+inline fm_status launch_tile(const TileArgs<T> &a, bool conv, hipStream_t stream) {
+    return conv ? launch_kind<T, true>(a, stream) : launch_kind<T, false>(a, stream);
+}
 
 // Largest tile (B*N elements) the engine supports for one precision.
 template <typename T> constexpr int max_tile_elems() {
     return sizeof(T) == 4 ? 16384 : 8192;
 }
 
-// Launch shape of a length-2^LOGN pass.  A thread holds 32 complex64 (16
-// complex128) elements by default.  Complex64 passes of 2-256 and of
-// 2048-8192 points hold 16 with twice the threads instead: the tile (and its
-// LDS) is unchanged, registers drop to ~90-125 per thread and a CU runs twice
-// the waves.  Up to 256 points the stage count is the same either way; at
-// 2048-8192 the extra waves pay for the extra stage; at 512 and 1024 points
-// the 32-element shape's one LDS exchange wins (measured on the uneven batch,
-// the Kron modes and the 2048-point Bluestein spectrum pass).
-template <typename T, int LOGN> struct PassCfg {
-    // (16384 points would need 1024 threads at <= 128 registers: it spills)
-    static constexpr bool e16 =
-        sizeof(T) == 4 && ((LOGN >= 11 && LOGN <= 13) || (LOGN >= 1 && LOGN <= 8));
-    static constexpr int LE = e16 ? 4 : -1;
-    static constexpr int NT =
-        e16 ? 512 : ((sizeof(T) == 4 ? LOGN >= 14 : LOGN >= 13) ? 512 : 256);
+// Launch shapes of a length-2^logn pass: elements per thread (2^le) and threads
+// per tile.  Strided and transposed sides want several sequences per tile (a
+// row segment of B elements, 8 of them 64 bytes of complex64); contiguous
+// sequences do not, and run better as many small tiles, whose load, exchange
+// and store phases overlap on a CU.  Where a launch has too few elements to give
+// every CU a tile of the large shapes, fewer elements per thread (shorter
+// chains of dependent butterflies and twiddle products) and smaller tiles cut
+// its latency.
+//   SHAPE_WIDE        strided or transposed sides
+//   SHAPE_ROW         contiguous sides
+//   SHAPE_SMALL_WIDE  the same for at most 2^19 elements,
+//   SHAPE_SMALL_ROW   and for at most 2^20
+// Measured (us, fft / spectrum pass; MI355X), shape = elements x threads:
+//   contiguous complex64      one shape for all before   ROW            SMALL_ROW
+//   1024 x 32768               32x256  111 / 142     16x128 102 / 120
+//   2048 x 16384               16x512  113 / 152     16x128 104 / 127
+//   4096 x 8192                16x512  109 / 149     16x256 102 / 128
+//   256 x 131072               16x512  104 / 118     16x256  99 / 107
+//   1024 x 16                  32x256  8.6 / 12.6                  8x128 4.5 / 6.5
+//   256 x 1024                 16x512  6.2 / 8.8                   8x64  4.1 / 5.3
+//   4096 x 4                   16x512  7.3 / 11.3                  8x512 5.3 / 8.2
+//   four-step 2^18 complex64, 512-point columns / rows
+//   32 columns                 32x256   32 / 40      8x512 28 (B = 8), 8x256 36
+//   1 column                   32x256   11 / 14      8x256 5.5 / 6.3
+//   contiguous complex128 1024 x 16  16x256 6.7 / 10.1   8x128 4.9 / 6.8
+enum PassShape { SHAPE_WIDE = 0, SHAPE_ROW = 1, SHAPE_SMALL_WIDE = 2, SHAPE_SMALL_ROW = 3 };
+constexpr int64_t kSmallWide = int64_t(1) << 19, kSmallRow = int64_t(1) << 20;
+
+template <typename T> constexpr int pass_le(int logn, int shape) {
+    const bool small = shape == SHAPE_SMALL_WIDE || shape == SHAPE_SMALL_ROW;
+    if (sizeof(T) == 4) {
+        if (logn == 0 || logn >= 14) return 5;
+        if (logn <= 6) return shape == SHAPE_WIDE ? 4 : 3;
+        if (logn <= 8) return small ? 3 : 4;
+        if (logn == 9) return 3;
+        if (logn == 10) return shape == SHAPE_WIDE ? 5 : (shape == SHAPE_SMALL_ROW ? 3 : 4);
+        if (logn <= 12) return shape == SHAPE_SMALL_ROW ? 3 : 4;
+        return 4;
+    }
+    if (logn == 0 || logn >= 12) return 4;
+    if (logn <= 8 && shape == SHAPE_SMALL_ROW) return 2;
+    if (logn <= 7) return 3;
+    if (logn <= 9) return shape == SHAPE_WIDE ? 4 : 3;
+    return shape == SHAPE_WIDE || shape == SHAPE_SMALL_WIDE ? 4 : 3;
+}
+
+template <typename T> constexpr int pass_nt(int logn, int shape) {
+    const bool small = shape == SHAPE_SMALL_WIDE || shape == SHAPE_SMALL_ROW;
+    const bool row = shape == SHAPE_ROW || shape == SHAPE_SMALL_ROW;
+    if (sizeof(T) == 4) {
+        if (logn == 0) return 256;
+        if (logn <= 6) return small ? 64 : 256;
+        if (logn == 7) return !small ? 256 : (row ? 64 : 128);
+        if (logn == 8) return shape == SHAPE_SMALL_ROW ? 64 : 256;
+        if (logn == 9) return shape == SHAPE_WIDE ? 512 : (shape == SHAPE_SMALL_ROW ? 128 : 256);
+        if (logn == 10) return row ? 128 : 256;
+        if (logn == 11) return !row ? 512 : (small ? 256 : 128);
+        if (logn == 12) return shape == SHAPE_ROW ? 256 : 512;
+        return 512;
+    }
+    if (logn == 0) return 256;
+    if (logn <= 6) return small ? 64 : 256;
+    if (logn == 7) return !small ? 256 : (row ? 64 : 128);
+    if (logn == 8) return shape == SHAPE_SMALL_ROW ? 64 : 256;
+    if (logn == 9) return !row ? 256 : (small ? 64 : 128);
+    if (logn == 10) return row ? 128 : 256;
+    return logn >= 13 ? 512 : 256;
+}
+
+template <typename T, int LOGN, int SHAPE> struct PassCfg {
+    static constexpr int LE = pass_le<T>(LOGN, SHAPE);
+    static constexpr int NT = pass_nt<T>(LOGN, SHAPE);
 };
 
-// Sequences per tile of the pass kernel for a length-2^logN transform.
-template <typename T> inline int tile_batch(int logN) {
-    const int loge = sizeof(T) == 4 ? 5 : 4;
-    const int lognt = (sizeof(T) == 4 ? logN >= 14 : logN >= 13) ? 9 : 8;
-    const int logb = lognt + loge - logN;
-    return logb > 0 ? (1 << logb) : 1;
+// Sequences per tile of a shape.
+template <typename T> inline int pass_batch(int logn, int shape) {
+    return (pass_nt<T>(logn, shape) << pass_le<T>(logn, shape)) >> logn;
 }
 
 }  // namespace fm

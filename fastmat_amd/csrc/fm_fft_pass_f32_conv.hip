@@ -1,0 +1,6 @@
+// Spectrum pass kernels of complex64 (see fm_fft_launch.hpp).
+#include "fm_fft_launch.hpp"
+
+namespace fm {
+template fm_status launch_kind<float, true>(const TileArgs<float> &, hipStream_t);
+}  // namespace fm

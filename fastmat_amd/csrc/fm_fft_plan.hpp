@@ -57,12 +57,20 @@ template <typename T> inline bool fits_idx32(const TileArgs<T> &a, int64_t N) {
              below(double(O1) * a.mid_os + double(N1) * a.mid_gn + double(J1) * a.mid_gj)));
 }
 
-// Fill in the tile shape (batch, tile count, log2 J) of a pass.
-template <typename T> inline fm_status normalize_pass(TileArgs<T> &a) {
+// Shape of a pass by its sides and size (see PassShape).
+template <typename T> inline int pick_shape(const TileArgs<T> &a, bool sized) {
+    const bool wide = a.seqfast_in || a.seqfast_out;
+    const int64_t elems = (a.O * a.J) << a.logN;
+    if (wide) return sized && elems <= kSmallWide ? SHAPE_SMALL_WIDE : SHAPE_WIDE;
+    return sized && elems <= kSmallRow ? SHAPE_SMALL_ROW : SHAPE_ROW;
+}
+
+// Fill in the tiling (sequences per tile, tile count, log2 J) of a pass.
+template <typename T> inline fm_status normalize_pass(TileArgs<T> &a, int B) {
     const int maxlog = sizeof(T) == 4 ? 14 : 13;
     FM_REQUIRE(a.logN >= 0 && a.logN <= maxlog, FM_ERR_VALUE,
                "sub-transform length 2^%d exceeds the tile limit", a.logN);
-    a.B = tile_batch<T>(a.logN);
+    a.B = B;
     a.ntiles = ceil_div(a.O * a.J, a.B);
     a.logJ = is_pow2(a.J) ? ilog2(a.J) : -1;
     if (a.o_group > 1 && ((a.J % a.B) != 0 || (a.O % a.o_group) != 0)) a.o_group = 1;
