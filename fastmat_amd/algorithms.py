@@ -29,6 +29,7 @@ import torch
 
 from . import _device as D
 from . import _lib
+from .circulant import Circulant, Toeplitz
 from .matrix import Matrix
 
 
@@ -151,11 +152,38 @@ class _Shrinkage(Algorithm):
             raise TypeError("%s needs a floating-point problem, got %s" % (self._name, w))
         return w
 
-    def _step(self, B, X, Y, Step, L, alpha, betas, counter, wdt):
+    def _fused(self, wdt, k):
+        """(plan, workspace) of the one-call step (fm_conv_shrink_step), or
+        None: a one-level Circulant or Toeplitz whose products have the
+        iterate's dtype."""
+        A = self.fmatA
+        if type(A) not in (Circulant, Toeplitz) or A._multi is not None or k < 1:
+            return None
+        if A.compute_dtype(wdt) != wdt or D.promote(wdt, A._minType) != wdt:
+            return None
+        h = A.plan_handle(wdt)
+        need = ctypes.c_int64()
+        try:
+            _lib.call("fm_conv_shrink_workspace_size", h, k, ctypes.byref(need))
+        except NotImplementedError:
+            return None
+        return h, D.workspace(need.value)
+
+    def _step(self, B, X, Y, Step, L, alpha, betas, counter, wdt, fused=None, keep_step=True):
         """One iteration on the device: Y is the point the gradient is taken
-        at (X itself for ISTA)."""
+        at (X itself for ISTA).  The fused step writes Step only where
+        keep_step asks for it (nothing reads it between steps)."""
         A = self.fmatA
         k = X.shape[0]
+        if fused is not None:
+            h, ws = fused
+            _lib.call("fm_conv_shrink_step", h, _lib.ptr(Y), _lib.ptr(B), k, float(L),
+                      float(alpha), _lib.ptr(X), _lib.ptr(Step) if keep_step else None,
+                      _lib.ptr(Y) if self._momentum else None,
+                      _lib.ptr(betas) if betas is not None else None,
+                      _lib.ptr(counter) if counter is not None else None,
+                      _lib.ptr(ws), ws.numel(), D.stream())
+            return
         F = A._apply(Y, False)
         if D.np_dtype(F.dtype) != wdt:
             F = F.to(D.torch_dtype(wdt))
@@ -204,32 +232,44 @@ class _Shrinkage(Algorithm):
                 t = (1 + np.sqrt(1 + 4 * t ** 2)) / 2
                 bl.append((t_old - 1) / t)
             betas = torch.tensor(bl, dtype=torch.float64, device=X.device)
-            counter = torch.zeros(1, dtype=torch.int64, device=X.device)
+            # the step index, and the fused step's count of finished workgroups
+            counter = torch.zeros(2, dtype=torch.int64, device=X.device)
+        fused = self._fused(wdt, k)
         callbacks = self.cbStep is not None or self.cbTrace is not None
         steps = int(self.numMaxSteps)
         self.numStep = 0
-        self._step(Bd, X, Y, Step, self.numL, alpha, betas, counter, wdt)
+
+        def step(keep_step=True):
+            self._step(Bd, X, Y, Step, self.numL, alpha, betas, counter, wdt, fused, keep_step)
+
+        step(callbacks or fused is None or steps == 1)
         if callbacks:
             self._expose(X, Step, on_device)
             self.handleCallback(self.cbStep)
             self.handleCallback(self.cbTrace)
             for self.numStep in range(1, steps):
-                self._step(Bd, X, Y, Step, self.numL, alpha, betas, counter, wdt)
+                step()
                 self._expose(X, Step, on_device)
                 self.handleCallback(self.cbStep)
                 self.handleCallback(self.cbTrace)
         elif steps > 1:
-            graph = torch.cuda.CUDAGraph()
-            cur = torch.cuda.current_stream()
-            side = torch.cuda.Stream()
-            side.wait_stream(cur)
-            with torch.cuda.stream(side):
-                with torch.cuda.graph(graph, stream=side):
-                    self._step(Bd, X, Y, Step, self.numL, alpha, betas, counter, wdt)
-            cur.wait_stream(side)
-            for self.numStep in range(1, steps):
-                graph.replay()
-            del graph
+            # one step captured and replayed; a fused run ends with an eager
+            # step that writes Step
+            last = steps - 1 if fused is not None else steps
+            if last > 1:
+                graph = torch.cuda.CUDAGraph()
+                cur = torch.cuda.current_stream()
+                side = torch.cuda.Stream()
+                side.wait_stream(cur)
+                with torch.cuda.stream(side):
+                    with torch.cuda.graph(graph, stream=side):
+                        step(keep_step=fused is None)
+                cur.wait_stream(side)
+                for self.numStep in range(1, last):
+                    graph.replay()
+                del graph
+            for self.numStep in range(last, steps):
+                step()
         res = torch.where(X != 0, Step, X)
         self._expose(X, Step, on_device)
         if on_device:

@@ -224,7 +224,7 @@ template <typename T> struct TileArgs {
     // optional residual epilogue (target != NULL): the store writes
     // out_scale * (u - t) with t read from `target` at the output's position
     // (same layout as y), and the tile's sum of |u - t|^2 over the stored
-    // elements goes to res_part[res_base + tile] (FP64)
+    // elements goes to res_part[res_base + tile] (FP64) unless res_part is NULL
     const cpx<T> *target;
     double *res_part;
     int64_t res_base;
@@ -554,14 +554,22 @@ __device__ __forceinline__ void tile_residual_sum(const TileArgs<T> &a, int64_t 
     __syncthreads();  // red is read before the LDS is written again
 }
 
+// Epilogue of a pass's store: none (plain stores), or an object whose
+// store<Ix, R>(idx, ok, u) takes over R elements u at offsets idx (those with
+// ok set) of the output's layout; it is called for a few elements at a time
+// so that it can load all of them before its first store.
+struct PlainStore {};
+constexpr int kEpilogueElems = 8;
+
 // Store the last stage's outputs of one tile: v[e*RL + r] holds element
 // i + r*N/RL (RL = 2^LOGRL, the radix of the stage that produced them) of
 // sequence b in mapping cur_sf; re-stage through LDS when the store wants the
 // other mapping, then apply the enclosing four-step twiddle / post-multiply /
 // conj / scale and write, cropping at m_valid.
-template <typename T, int LOGN, int NT, int LOGRL, bool I32 = false, int LE = -1>
+template <typename T, int LOGN, int NT, int LOGRL, bool I32 = false, int LE = -1,
+          typename EP = PlainStore>
 __device__ __forceinline__ void fft_tile_store(const TileArgs<T> &a, int64_t tile, cpx<T> *v,
-                                               cpx<T> *lds, bool cur_sf) {
+                                               cpx<T> *lds, bool cur_sf, const EP &ep = EP()) {
     using S = TileShape<T, LOGN, NT, LE>;
     using Ix = IdxT<I32>;
     constexpr int E = S::E;
@@ -624,6 +632,22 @@ __device__ __forceinline__ void fft_tile_store(const TileArgs<T> &a, int64_t til
                 if (gidx < mv) v[e * RL + r] = cmul(v[e * RL + r], ldg(a.post, gidx));
             }
         }
+        if constexpr (!std::is_same<EP, PlainStore>::value) {
+            constexpr int C = RL < kEpilogueElems ? RL : kEpilogueElems;
+#pragma unroll
+            for (int r0 = 0; r0 < RL; r0 += C) {
+                Ix idx[C];
+                bool ok[C];
+#pragma unroll
+                for (int r = 0; r < C; ++r) {
+                    const Ix n = Ix(i + (r0 + r) * NRL);
+                    ok[r] = n * out_gn + sp.j * out_gj < mv;
+                    idx[r] = sp.out_base + n * out_ns;
+                }
+                ep.template store<Ix, C>(idx, ok, v + e * RL + r0);
+            }
+            continue;
+        }
 #pragma unroll
         for (int r = 0; r < RL; ++r) {
             const Ix n = Ix(i + r * NRL);
@@ -633,7 +657,7 @@ __device__ __forceinline__ void fft_tile_store(const TileArgs<T> &a, int64_t til
             if (a.conj_out) u = conj(u);
             if (a.target) {
                 const cpx<T> d = u - ldg(a.target, Ix(sp.out_base + n * out_ns));
-                res2 += double(d.x) * double(d.x) + double(d.y) * double(d.y);
+                if (a.res_part) res2 += double(d.x) * double(d.x) + double(d.y) * double(d.y);
                 u = d;
             }
             if (a.stream_out & 1)
@@ -642,15 +666,16 @@ __device__ __forceinline__ void fft_tile_store(const TileArgs<T> &a, int64_t til
                 stg(a.y, Ix(sp.out_base + n * out_ns), scale(u, a.out_scale));
         }
     }
-    if (a.target) tile_residual_sum<T, NT>(a, tile, res2, lds);
+    if (a.target && a.res_part) tile_residual_sum<T, NT>(a, tile, res2, lds);
 }
 
 // Everything after the stage-0 loads of one tile: conj / pre-multiply, the
 // transform (conv: forward, spectrum, inverse), twiddle / post-multiply and
 // the stores.  `lds` holds B * (N + N/32 + 1) elements.
-template <typename T, int LOGN, int NT, bool CONV, bool I32 = false, int LE = -1>
+template <typename T, int LOGN, int NT, bool CONV, bool I32 = false, int LE = -1,
+          typename EP = PlainStore>
 __device__ __forceinline__ void fft_tile_compute(const TileArgs<T> &a, int64_t tile, cpx<T> *v,
-                                                 cpx<T> *lds) {
+                                                 cpx<T> *lds, const EP &ep = EP()) {
     using S = TileShape<T, LOGN, NT, LE>;
     using Ix = IdxT<I32>;
     constexpr int LOGE = S::LOGE;
@@ -740,13 +765,14 @@ __device__ __forceinline__ void fft_tile_compute(const TileArgs<T> &a, int64_t t
                         cpx<T> u = mk(T(0), T(0));
                         if (g < mv) {
                             const cpx<T> d = v[e * RF + r] - ldg(a.mid_t, Ix(tb + g));
-                            res2 += double(d.x) * double(d.x) + double(d.y) * double(d.y);
+                            if (a.res_part)
+                                res2 += double(d.x) * double(d.x) + double(d.y) * double(d.y);
                             u = scale(d, a.mid_scale);
                         }
                         v[e * RF + r] = u;
                     }
                 }
-                tile_residual_sum<T, NT>(a, tile, res2, lds);
+                if (a.res_part) tile_residual_sum<T, NT>(a, tile, res2, lds);
             } else {
 #pragma unroll
                 for (int e = 0; e < NBF; ++e) {
@@ -769,14 +795,16 @@ __device__ __forceinline__ void fft_tile_compute(const TileArgs<T> &a, int64_t t
         if (P::S > 1) cur_sf = false;
     }
 
-    fft_tile_store<T, LOGN, NT, LOGRL, I32, LE>(a, tile, v, lds, cur_sf);
+    fft_tile_store<T, LOGN, NT, LOGRL, I32, LE, EP>(a, tile, v, lds, cur_sf, ep);
 }
 
-template <typename T, int LOGN, int NT, bool CONV, bool I32 = false, int LE = -1>
-__device__ __forceinline__ void fft_pass_body(const TileArgs<T> &a, int64_t tile, cpx<T> *lds) {
+template <typename T, int LOGN, int NT, bool CONV, bool I32 = false, int LE = -1,
+          typename EP = PlainStore>
+__device__ __forceinline__ void fft_pass_body(const TileArgs<T> &a, int64_t tile, cpx<T> *lds,
+                                              const EP &ep = EP()) {
     cpx<T> v[TileShape<T, LOGN, NT, LE>::E];
     fft_tile_load<T, LOGN, NT, I32, LE>(a, tile, v);
-    fft_tile_compute<T, LOGN, NT, CONV, I32, LE>(a, tile, v, lds);
+    fft_tile_compute<T, LOGN, NT, CONV, I32, LE, EP>(a, tile, v, lds, ep);
 }
 
 template <typename T, int LOGN, int NT, bool CONV, bool I32, int LE = -1>
