@@ -29,28 +29,52 @@ SUPPORTED = tuple(_NP2T)
 
 def np_dtype(dt):
     """numpy dtype of a numpy dtype-like or torch dtype."""
+    if isinstance(dt, np.dtype):
+        return dt
+    r = _T2NP.get(dt)
+    if r is not None:
+        return r
     if isinstance(dt, torch.dtype):
-        if dt not in _T2NP:
-            raise TypeError("Unsupported data type %s" % dt)
-        return _T2NP[dt]
+        raise TypeError("Unsupported data type %s" % dt)
     return np.dtype(dt)
 
 
 def torch_dtype(dt):
-    dt = np_dtype(dt)
-    if dt not in _NP2T:
-        raise TypeError("Unsupported data type %s" % dt)
-    return _NP2T[dt]
+    t = _NP2T.get(np_dtype(dt))
+    if t is None:
+        raise TypeError("Unsupported data type %s" % np_dtype(dt))
+    return t
 
 
 def fm_type(dt):
     return _lib.NP_TO_FM[np_dtype(dt)]
 
 
+# Type rules are looked up on every apply of a small operand: their results, per
+# pair of types, are kept (the types are few).
+_promoted = {}
+_input_types = {}
+
+
 def promote(a, b):
     """numpy promotion (the reference's promotion table equals
     np.promote_types, core/types.pyx:418-453)."""
-    return np.promote_types(np_dtype(a), np_dtype(b))
+    r = _promoted.get((a, b))
+    if r is None:
+        r = _promoted[a, b] = np.promote_types(np_dtype(a), np_dtype(b))
+    return r
+
+
+def input_type(in_dtype, min_type, dtype, widen):
+    """torch type in which an operator of type `dtype` takes data of the torch
+    type `in_dtype` (Matrix._prepareInputArray, Matrix.pyx:1737-1817):
+    promote(input, minType), widened to the output's type where asked."""
+    key = (in_dtype, min_type, dtype, widen)
+    r = _input_types.get(key)
+    if r is None:
+        fin = promote(in_dtype, min_type)
+        r = _input_types[key] = torch_dtype(promote(fin, dtype) if widen else fin)
+    return r
 
 
 def safe_type_expansion(dtype):
@@ -140,8 +164,16 @@ def empty(k, n, dtype):
     return torch.empty((k, n), dtype=torch_dtype(dtype), device=device())
 
 
+# Raw handle of the current stream without building a Stream object (2 us of a
+# small apply); older torch versions lack it.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream():
-    return _lib.stream_handle(device())
+    """hipStream_t of torch's current stream on the device, as an address."""
+    if _raw_stream is None:
+        return _lib.stream_handle(device())
+    return _raw_stream(device().index)
 
 
 def ld(t):

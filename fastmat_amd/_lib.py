@@ -185,20 +185,27 @@ def check(status):
     raise FastmatAmdError(msg or "fastmat_amd error %d" % status)
 
 
+_functions = {}
+
+
 def call(name, *args):
-    lib = load()
-    check(getattr(lib, name)(*args))
+    f = _functions.get(name)
+    if f is None:
+        f = _functions[name] = getattr(load(), name)
+    status = f(*args)
+    if status:
+        check(status)
 
 
 def stream_handle(device=None):
-    """hipStream_t of torch's current stream on `device`, as a c_void_p."""
+    """hipStream_t of torch's current stream on `device`, as an address."""
     import torch
-    s = torch.cuda.current_stream(device)
-    return ctypes.c_void_p(s.cuda_stream)
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def ptr(t):
-    return ctypes.c_void_p(t.data_ptr())
+    """Device address of a tensor's first element."""
+    return t.data_ptr()
 
 
 def dvec(z):

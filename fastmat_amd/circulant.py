@@ -79,7 +79,7 @@ class _ConvBase(Matrix):
         """Apply the native plan `h` to the (k, n) block X of its precision."""
         k, n = X.shape
         m = self.numCols if adjoint else self.numRows
-        Y = D.empty(k, m, X.dtype)
+        Y = X.new_empty((k, m))
         need = ctypes.c_int64()
         _lib.call("fm_conv_workspace_size", h, k, ctypes.byref(need))
         ws = D.workspace(need.value)

@@ -44,19 +44,21 @@ class _PlanCache:
         self._plans = {}
 
 
+_C64, _C128 = np.dtype(np.complex64), np.dtype(np.complex128)
+_PRECISION = {_C64: _lib.FM_COMPLEX64, _C128: _lib.FM_COMPLEX128}
+
+
 def precision_of(dtype):
     dt = D.np_dtype(dtype)
-    if dt == np.complex64:
-        return _lib.FM_COMPLEX64
-    if dt == np.complex128:
-        return _lib.FM_COMPLEX128
-    raise TypeError("Fourier-type operators compute in complex64 or complex128, not %s" % dt)
+    p = _PRECISION.get(dt)
+    if p is None:
+        raise TypeError("Fourier-type operators compute in complex64 or complex128, not %s" % dt)
+    return p
 
 
 def complex_of(dtype):
     """The complex dtype an operator computes in for a promoted dtype."""
-    dt = D.np_dtype(dtype)
-    return np.promote_types(dt, np.complex64)
+    return D.promote(dtype, _C64)
 
 
 class Fourier(Matrix):
@@ -119,7 +121,7 @@ class Fourier(Matrix):
             X = X.to(D.torch_dtype(cdt))
         h = self._plans.get(precision_of(cdt))
         k, n = X.shape
-        Y = D.empty(k, n, cdt)
+        Y = X.new_empty((k, n))
         need = ctypes.c_int64()
         _lib.call("fm_fourier_workspace_size", h, k, ctypes.byref(need))
         ws = D.workspace(need.value)

@@ -319,12 +319,9 @@ class Matrix:
 
     def _apply(self, X, adjoint):
         """Type promotion (Matrix._prepareInputArray) then the transform."""
-        fin = D.promote(X.dtype, self._minType)
-        fout = D.promote(fin, self.dtype)
-        if self._widenInputDatatype:
-            fin = fout
-        if D.np_dtype(X.dtype) != fin:
-            X = X.to(D.torch_dtype(fin))
+        t = D.input_type(X.dtype, self._minType, self.dtype, self._widenInputDatatype)
+        if X.dtype is not t:
+            X = X.to(t)
         return self._bwd(X) if adjoint else self._fwd(X)
 
     def _apply_into(self, X, Y, adjoint):
