@@ -155,9 +155,34 @@ def to_block(arr, required):
     block = t.t()
     if block.device != dev:
         block = block.to(dev, non_blocking=False)
-    if not block.is_contiguous():
-        block = block.contiguous()
-    return block, Boundary(kind, was1d, dev)
+    return contiguous_block(block), Boundary(kind, was1d, dev)
+
+
+# Row-major operands from this size on go through the library's transpose; torch's
+# strided copy costs the host less and is as fast below (2 MB complex128: 4.4 us).
+_TRANSPOSE_BYTES = 4 << 20
+
+
+def contiguous_block(block):
+    """The (k, n) view `block` as a contiguous tensor.  Columns of a large
+    row-major (n, k) array on the device go through the library's transpose
+    (complex64 2^18 x 32: 26 us, torch's strided copy 63 us); small ones, other
+    layouts, lazily conjugated or negated tensors and tensor subclasses through
+    torch."""
+    if block.is_contiguous():
+        return block
+    k, n = block.shape
+    esz = block.element_size()
+    if k * n * esz >= _TRANSPOSE_BYTES and type(block) is torch.Tensor:
+        s0, s1 = block.stride()
+        if (s0 == 1 and s1 >= k and block.dtype in _T2NP and block.device == device() and
+                not block.is_conj() and not block.is_neg() and
+                (esz < 16 or block.data_ptr() % 16 == 0)):
+            out = block.new_empty((k, n))
+            _lib.call("fm_transpose", esz, n, k, block.data_ptr(), s1, out.data_ptr(), n,
+                      stream())
+            return out
+    return block.contiguous()
 
 
 def empty(k, n, dtype):

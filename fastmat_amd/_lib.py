@@ -69,6 +69,7 @@ _PROTOTYPES = {
     "fm_kron_pair_apply": (_c_int, [_vp, _c_int, _vp, _c_i64, _vp, _vp, _c_i64, _vp]),
     "fm_diag_apply": (_c_int, [_c_int, _c_int, _c_i64, _vp, _vp, _c_i64, _vp, _c_i64, _c_i64,
                                _vp]),
+    "fm_transpose": (_c_int, [_c_int, _c_i64, _c_i64, _vp, _c_i64, _vp, _c_i64, _vp]),
     "fm_gather_rows": (_c_int, [_c_int, _c_i64, _vp, _vp, _c_i64, _vp, _c_i64, _c_i64, _vp]),
     "fm_scatter_rows": (_c_int, [_c_int, _c_i64, _vp, _vp, _c_i64, _vp, _c_i64, _c_i64, _c_i64,
                                  _vp]),

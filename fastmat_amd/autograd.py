@@ -30,7 +30,7 @@ from . import _device as D
 
 def _to_block(x):
     was1d = x.dim() == 1
-    X = (x.reshape(-1, 1) if was1d else x).t().contiguous()
+    X = D.contiguous_block((x.reshape(-1, 1) if was1d else x).t())
     return X, was1d
 
 
@@ -130,7 +130,7 @@ class _BatchConvMatvec(torch.autograd.Function):
         ctx.gen_complex = [g.is_complex() for g in gens]
         ctx.gen_dtype = [g.dtype for g in gens]
         ctx.tok = batch.load_generators(gens)
-        X = [x.t().contiguous() for x in xs]
+        X = [D.contiguous_block(x.t()) for x in xs]
         Y = batch.forward(X)
         ctx.batch = batch
         ctx.n = n
@@ -143,7 +143,7 @@ class _BatchConvMatvec(torch.autograd.Function):
         n = ctx.n
         saved = ctx.saved_tensors
         X, gens = saved[:n], saved[n:]
-        G = [g.t().contiguous() for g in gs]
+        G = [D.contiguous_block(g.t()) for g in gs]
         need_gen = any(ctx.needs_input_grad[1:1 + n])
         need_x = any(ctx.needs_input_grad[1 + n:])
         gx = [None] * n

@@ -381,6 +381,11 @@ fm_status fm_kron_conv_dense_apply(const fm_conv_plan *plan, int conj_circulant,
 fm_status fm_diag_apply(int dtype, int conj_d, int64_t n, const void *d,
                         const void *x, int64_t ldx, void *y, int64_t ldy,
                         int64_t k, void *stream);
+/* dst[c * ld_dst + i] = src[i * ld_src + c] for i < n, c < k, elements of 1, 2,
+ * 4, 8 or 16 bytes (16-byte ones 16-byte aligned): a row-major n x k array to
+ * column-major blocks.  src and dst must not overlap. */
+fm_status fm_transpose(int elem_bytes, int64_t n, int64_t k, const void *src,
+                       int64_t ld_src, void *dst, int64_t ld_dst, void *stream);
 /* y[i,:] = x[idx[i],:] for i < n_out (row gather; Permutation._forward /
  * _backward, Permutation.pyx:121-125, and Partial's row selection,
  * Partial.pyx:268-294).  idx: device int64. */
