@@ -2,9 +2,10 @@
 
 Forward scatters x into a zero-padded vector of the nested matrix's width at
 ``colSelection``, applies the matrix and gathers ``rowSelection``
-(Partial.pyx:268-280); backward mirrors it (:282-294).  Scatter and gather run
-as library kernels."""
+(Partial.pyx:268-280); backward mirrors it (:282-294).  Scatter (through the
+selection's inverse) and gather run as library kernels."""
 import numpy as np
+import torch
 
 from . import _device as D
 from . import _lib
@@ -89,11 +90,28 @@ class Partial(Matrix):
             t = self._dev[name] = D.as_tensor(_device_index(sel, size), np.int64)
         return t
 
+    def _inverse(self, name, sel):
+        """Row of the selection that lands on each row of the nested matrix's
+        operand, -1 for none (the last one of equal indices, as numpy's
+        indexed assignment leaves it)."""
+        t = self._dev.get("inv" + name)
+        if t is None:
+            M = self._content[0]
+            idx = self._idx(name, sel)
+            t = torch.full((M.numRows if name == "r" else M.numCols,), -1, dtype=torch.int64,
+                           device=idx.device)
+            t.scatter_reduce_(0, idx, torch.arange(idx.numel(), device=idx.device), "amax")
+            self._dev["inv" + name] = t
+        return t
+
     def _scatter(self, X, sel, name, n_full):
         k, n = X.shape
         Y = D.empty(k, n_full, X.dtype)
-        _lib.call("fm_scatter_rows", D.fm_type(X.dtype), n, _lib.ptr(self._idx(name, sel)),
-                  _lib.ptr(X), n, _lib.ptr(Y), n_full, n_full, k, D.stream())
+        if n == 0:
+            return Y.zero_()
+        _lib.call("fm_expand_rows", D.fm_type(X.dtype), n_full,
+                  _lib.ptr(self._inverse(name, sel)), _lib.ptr(X), n, _lib.ptr(Y), n_full, k,
+                  D.stream())
         return Y
 
     def _gather(self, X, sel, name):

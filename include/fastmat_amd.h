@@ -392,6 +392,10 @@ fm_status fm_transpose(int elem_bytes, int64_t n, int64_t k, const void *src,
 fm_status fm_gather_rows(int dtype, int64_t n_out, const int64_t *idx,
                          const void *x, int64_t ldx, void *y, int64_t ldy,
                          int64_t k, void *stream);
+/* y[i,:] = x[src[i],:] where src[i] >= 0, else 0, for i < n_out: Partial's
+ * zero-padded scatter from its inverse index, one write per row. */
+fm_status fm_expand_rows(int dtype, int64_t n_out, const int64_t *src, const void *x,
+                         int64_t ldx, void *y, int64_t ldy, int64_t k, void *stream);
 /* y = 0 (n_out rows); y[idx[i],:] = x[i,:] for i < n_in (Partial's
  * zero-padded scatter, Partial.pyx:270-276). */
 fm_status fm_scatter_rows(int dtype, int64_t n_in, const int64_t *idx,
