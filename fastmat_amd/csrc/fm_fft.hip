@@ -381,9 +381,10 @@ extern "C" fm_status fm_fourier_workspace_size(const fm_fourier_plan *p, int64_t
     return FM_SUCCESS;
 }
 
-extern "C" fm_status fm_fourier_apply(const fm_fourier_plan *p, int adjoint, const void *x,
-                                      int64_t ldx, void *y, int64_t ldy, int64_t k,
-                                      void *workspace, int64_t workspace_bytes, void *stream) {
+static fm_status fourier_apply(const fm_fourier_plan *p, int adjoint, const void *x, int64_t ldx,
+                               void *y, int64_t ldy, int64_t k, const void *pre,
+                               const void *post, void *workspace, int64_t workspace_bytes,
+                               void *stream) {
     FM_REQUIRE(p != nullptr, FM_ERR_VALUE, "plan is NULL");
     FM_REQUIRE(k >= 0, FM_ERR_VALUE, "negative column count");
     if (k == 0) return FM_SUCCESS;
@@ -402,12 +403,32 @@ extern "C" fm_status fm_fourier_apply(const fm_fourier_plan *p, int adjoint, con
     io.n_in = p->N; io.m_out = p->N;
     io.conj_io = adjoint ? 1 : 0;
     io.work = workspace;
+    io.pre = pre;
+    io.post = post;
     if (p->bluestein) {
         io.pre = p->chirp;
         io.post = p->chirp;
         io.D = p->D;
     }
     return run_pipeline_any(p->geo, io, as_stream(stream), &p->lanes);
+}
+
+extern "C" fm_status fm_fourier_apply(const fm_fourier_plan *p, int adjoint, const void *x,
+                                      int64_t ldx, void *y, int64_t ldy, int64_t k,
+                                      void *workspace, int64_t workspace_bytes, void *stream) {
+    return fourier_apply(p, adjoint, x, ldx, y, ldy, k, nullptr, nullptr, workspace,
+                         workspace_bytes, stream);
+}
+
+extern "C" fm_status fm_fourier_apply_diag(const fm_fourier_plan *p, int adjoint, const void *pre,
+                                           const void *post, const void *x, int64_t ldx, void *y,
+                                           int64_t ldy, int64_t k, void *workspace,
+                                           int64_t workspace_bytes, void *stream) {
+    FM_REQUIRE(p != nullptr, FM_ERR_VALUE, "plan is NULL");
+    FM_REQUIRE(!p->bluestein, FM_ERR_NOT_IMPLEMENTED,
+               "diagonals fused with a Fourier matrix need a power-of-two order");
+    return fourier_apply(p, adjoint, x, ldx, y, ldy, k, pre, post, workspace, workspace_bytes,
+                         stream);
 }
 
 extern "C" fm_status fm_fourier_apply_strided(const fm_fourier_plan *p, int adjoint,

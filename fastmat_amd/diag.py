@@ -42,6 +42,15 @@ class Diag(Matrix):
             t = self._dev[dt] = D.as_tensor(self._vecD, dt)
         return t
 
+    def _table(self, dt, conj):
+        """The diagonal on the device in the complex type dt, or its conjugate."""
+        if not conj or self._vecD.dtype.kind != "c":
+            return self._d(dt)
+        t = self._dev.get((dt, "conj"))
+        if t is None:
+            t = self._dev[dt, "conj"] = D.as_tensor(self._vecD.conj(), dt)
+        return t
+
     def _run(self, X, conj_d):
         dt = D.promote(X.dtype, self.dtype)
         if D.np_dtype(X.dtype) != dt:

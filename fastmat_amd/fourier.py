@@ -129,6 +129,29 @@ class Fourier(Matrix):
                   None if ws is None else _lib.ptr(ws), need.value, D.stream())
         return Y
 
+    def _diag_ok(self, X):
+        """True when diagonals can run inside the transform of X: a
+        power-of-two order (Bluestein's chirps take their place otherwise) and
+        data that is already of the compute type."""
+        return (self._order & (self._order - 1) == 0 and
+                D.np_dtype(X.dtype) == self.compute_dtype(X.dtype) and
+                D.promote(X.dtype, self._minType) == D.np_dtype(X.dtype))
+
+    def _run_diag(self, X, adjoint, pre, post):
+        """diag(post) F diag(pre) X, or its conjugates around F^H (pre, post:
+        device vectors of X's type, or None); see _diag_ok."""
+        h = self._plans.get(precision_of(X.dtype))
+        k, n = X.shape
+        Y = X.new_empty((k, n))
+        need = ctypes.c_int64()
+        _lib.call("fm_fourier_workspace_size", h, k, ctypes.byref(need))
+        ws = D.workspace(need.value)
+        _lib.call("fm_fourier_apply_diag", h, int(adjoint),
+                  None if pre is None else _lib.ptr(pre), None if post is None else _lib.ptr(post),
+                  _lib.ptr(X), n, _lib.ptr(Y), n, k, None if ws is None else _lib.ptr(ws),
+                  need.value, D.stream())
+        return Y
+
     def _apply_views(self, X, Y, adjoint):
         cdt = self.compute_dtype(X.dtype)
         if D.np_dtype(X.dtype) != cdt or D.np_dtype(Y.dtype) != cdt:

@@ -7,7 +7,9 @@ scalars multiply (:101-105); dtype = promote(factors, scalars) expanded by
 import numpy as np
 
 from . import _device as D
-from .matrix import Matrix, scale_block
+from .diag import Diag
+from .fourier import Fourier
+from .matrix import Hermitian, Matrix, scale_block
 
 
 class Product(Matrix):
@@ -65,16 +67,10 @@ class Product(Matrix):
         return X
 
     def _fwd(self, X):
-        X = self._prep(X, False)
-        for f in reversed(self._content):
-            X = f._apply(X, False)
-        return X
+        return _apply_chain(self._content[::-1], self._prep(X, False), False)
 
     def _bwd(self, X):
-        X = self._prep(X, np.iscomplexobj(self._scalar))
-        for f in self._content:
-            X = f._apply(X, True)
-        return X
+        return _apply_chain(self._content, self._prep(X, np.iscomplexobj(self._scalar)), True)
 
     def _reference(self):
         dt = np.promote_types(np.float64, self.dtype)
@@ -82,3 +78,52 @@ class Product(Matrix):
         for f in self._content[-2::-1]:
             res = f.reference().dot(res)
         return res
+
+
+def _apply_chain(factors, X, adjoint):
+    """The factors (their adjoints) applied to X one after another, the first in
+    the sequence first.  A Fourier factor takes neighbouring Diag factors into
+    its passes (fm_fourier_apply_diag): they multiply as the transform reads and
+    writes, instead of a pass over the data each."""
+    i = 0
+    while i < len(factors):
+        fused = _fourier_with_diags(factors, i, X, adjoint)
+        if fused is None:
+            X = factors[i]._apply(X, adjoint)
+            i += 1
+        else:
+            X, i = fused
+    return X
+
+
+def _fourier_with_diags(factors, i, X, adjoint):
+    """(result, next index) of a Diag / Fourier / Diag run starting at i that
+    has a Fourier and at least one Diag, or None."""
+    pre = factors[i] if type(factors[i]) is Diag else None
+    f = i + (pre is not None)
+    if f >= len(factors):
+        return None
+    F, flip = _as_fourier(factors[f])
+    post = factors[f + 1] if f + 1 < len(factors) and type(factors[f + 1]) is Diag else None
+    if F is None or (pre is None and post is None) or not F._diag_ok(X):
+        return None
+    dt = D.np_dtype(X.dtype)
+    if not all(d is None or (D.promote(dt, d.dtype) == dt and D.promote(dt, d._minType) == dt)
+               for d in (pre, post)):
+        return None
+    # the transform conjugates its tables when it is an adjoint one; a Diag's
+    # adjoint is its conjugate
+    inverse = adjoint != flip
+    Y = F._run_diag(X, inverse, None if pre is None else pre._table(dt, inverse != adjoint),
+                    None if post is None else post._table(dt, inverse != adjoint))
+    return Y, f + 1 + (post is not None)
+
+
+def _as_fourier(f):
+    """(Fourier, False) for a Fourier matrix, (Fourier, True) for its Hermitian,
+    (None, False) otherwise."""
+    if type(f) is Fourier:
+        return f, False
+    if type(f) is Hermitian and type(f._nested) is Fourier:
+        return f._nested, True
+    return None, False

@@ -107,6 +107,14 @@ fm_status fm_fourier_apply(const fm_fourier_plan *plan, int adjoint,
                            const void *x, int64_t ldx, void *y, int64_t ldy,
                            int64_t k, void *workspace, int64_t workspace_bytes,
                            void *stream);
+/* fm_fourier_apply with diagonal factors in its passes (power-of-two orders):
+ * y = diag(post) F diag(pre) x, or with adjoint != 0
+ * y = diag(conj post) F^H diag(conj pre) x; pre, post: order entries of the
+ * plan's precision, or NULL. */
+fm_status fm_fourier_apply_diag(const fm_fourier_plan *plan, int adjoint, const void *pre,
+                                const void *post, const void *x, int64_t ldx, void *y,
+                                int64_t ldy, int64_t k, void *workspace,
+                                int64_t workspace_bytes, void *stream);
 /* Mode-wise DFT along a strided axis (Kron mode application,
  * Kron.pyx:267-303): vectors v[i] = x[(o*N + i)*inner + j]; requires a
  * single-pass plan (N up to the LDS tile size). */
