@@ -165,14 +165,14 @@ class _ConvBase(Matrix):
         set from device generators (fm_conv_set_generator); the matrix's own
         plan keeps the spectrum of the constructor's generator."""
         if getattr(self, "_gplans", None) is None:
-            def clone(prec):
-                h = ctypes.c_void_p()
-                _lib.call("fm_conv_plan_clone", self._plans.get(prec), D.stream(),
-                          ctypes.byref(h))
-                return h
-            self._gplans = _PlanCache(clone, "fm_conv_plan_destroy")
+            self._gplans = _PlanCache(self._clone_plan, "fm_conv_plan_destroy")
             self._gtokens = {}
         return self._gplans.get(precision_of(cdt))
+
+    def _clone_plan(self, prec):
+        h = ctypes.c_void_p()
+        _lib.call("fm_conv_plan_clone", self._plans.get(prec), D.stream(), ctypes.byref(h))
+        return h
 
     def load_generator(self, gen, cdt):
         """Make the private plan of precision `cdt` the operator of the device

@@ -13,6 +13,7 @@ twiddles), complex128 otherwise.  The reference always reports complex128
 complex64 input under numpy 2.
 """
 import ctypes
+import weakref
 
 import numpy as np
 
@@ -23,17 +24,20 @@ from .matrix import Matrix
 
 class _PlanCache:
     """Per-precision native plans, created on first use and destroyed with
-    the owning matrix."""
+    the owning matrix.  ``create`` is a method of the owner, held weakly: the
+    owner then goes, and frees its device memory, with its last reference, not
+    whenever the cycle collector runs (inside a stream capture such a free ends
+    the capture with an error)."""
 
     def __init__(self, create, destroy):
-        self._create = create
+        self._create = weakref.WeakMethod(create)
         self._destroy = destroy
         self._plans = {}
 
     def get(self, prec):
         h = self._plans.get(prec)
         if h is None:
-            h = self._plans[prec] = self._create(prec)
+            h = self._plans[prec] = self._create()(prec)
         return h
 
     def drop(self):
