@@ -45,6 +45,8 @@ _PROTOTYPES = {
                                   _vp]),
     "fm_fourier_apply_diag": (_c_int, [_vp, _c_int, _vp, _vp, _vp, _c_i64, _vp, _c_i64, _c_i64,
                                        _vp, _c_i64, _vp]),
+    "fm_fourier_apply_select": (_c_int, [_vp, _c_int, _vp, _vp, _vp, _vp, _vp, _c_i64, _vp, _c_i64,
+                                         _c_i64, _vp, _c_i64, _vp]),
     "fm_fourier_apply_strided": (_c_int, [_vp, _c_int, _vp, _vp, _c_i64, _c_i64, _vp]),
     "fm_fourier_plan_destroy": (_c_int, [_vp]),
     "fm_circulant_plan_create": (_c_int, [_c_int, _c_i64, _vp, _vp, _pp]),

@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "fm_fft_plan.hpp"
+#include "fm_select.hpp"
 
 namespace fm {
 
@@ -384,12 +385,12 @@ extern "C" fm_status fm_fourier_workspace_size(const fm_fourier_plan *p, int64_t
 static fm_status fourier_apply(const fm_fourier_plan *p, int adjoint, const void *x, int64_t ldx,
                                void *y, int64_t ldy, int64_t k, const void *pre,
                                const void *post, void *workspace, int64_t workspace_bytes,
-                               void *stream) {
+                               void *stream, const int *in = nullptr, const int *out = nullptr) {
     FM_REQUIRE(p != nullptr, FM_ERR_VALUE, "plan is NULL");
     FM_REQUIRE(k >= 0, FM_ERR_VALUE, "negative column count");
     if (k == 0) return FM_SUCCESS;
     FM_REQUIRE(x && y, FM_ERR_VALUE, "NULL data pointer");
-    FM_REQUIRE(ldx >= p->N && ldy >= p->N, FM_ERR_VALUE,
+    FM_REQUIRE((in || ldx >= p->N) && (out || ldy >= p->N), FM_ERR_VALUE,
                "leading dimensions (%lld, %lld) below the order %lld", (long long)ldx,
                (long long)ldy, (long long)p->N);
     int64_t need = 0;
@@ -410,7 +411,25 @@ static fm_status fourier_apply(const fm_fourier_plan *p, int adjoint, const void
         io.post = p->chirp;
         io.D = p->D;
     }
+    if (in || out)
+        return p->prec == FM_COMPLEX64
+                   ? run_selected<float>(p->geo, io, in, out, as_stream(stream), &p->lanes)
+                   : run_selected<double>(p->geo, io, in, out, as_stream(stream), &p->lanes);
     return run_pipeline_any(p->geo, io, as_stream(stream), &p->lanes);
+}
+
+extern "C" fm_status fm_fourier_apply_select(const fm_fourier_plan *p, int adjoint,
+                                             const void *pre, const void *post,
+                                             const int32_t *in_index, const int32_t *out_index,
+                                             const void *x, int64_t ldx, void *y, int64_t ldy,
+                                             int64_t k, void *workspace,
+                                             int64_t workspace_bytes, void *stream) {
+    FM_REQUIRE(p != nullptr, FM_ERR_VALUE, "plan is NULL");
+    FM_REQUIRE(!p->bluestein || (!pre && !post), FM_ERR_NOT_IMPLEMENTED,
+               "diagonals fused with a Fourier matrix need a power-of-two order");
+    FM_REQUIRE(ldx >= 1 && ldy >= 1, FM_ERR_VALUE, "leading dimensions below one");
+    return fourier_apply(p, adjoint, x, ldx, y, ldy, k, pre, post, workspace, workspace_bytes,
+                         stream, in_index, out_index);
 }
 
 extern "C" fm_status fm_fourier_apply(const fm_fourier_plan *p, int adjoint, const void *x,

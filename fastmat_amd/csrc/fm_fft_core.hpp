@@ -498,10 +498,16 @@ __device__ __forceinline__ int64_t tile_first_seq(const TileArgs<T> &a, int64_t 
     return o * a.J + (jb << LOGB);
 }
 
+// Where a pass's input elements come from: their own places (PlainLoad), or an
+// object whose table(e) names the element of the column to read in place of
+// element e, negative for a zero; a NULL table is the plain load.
+struct PlainLoad {};
+
 // Stage-0 inputs of one tile straight from global memory (zero outside the
 // valid range); only loads, so a caller can issue them ahead of compute.
-template <typename T, int LOGN, int NT, bool I32 = false, int LE = -1>
-__device__ __forceinline__ void fft_tile_load(const TileArgs<T> &a, int64_t tile, cpx<T> *v) {
+template <typename T, int LOGN, int NT, bool I32 = false, int LE = -1, typename LP = PlainLoad>
+__device__ __forceinline__ void fft_tile_load(const TileArgs<T> &a, int64_t tile, cpx<T> *v,
+                                              const LP &lp = LP()) {
     using S = TileShape<T, LOGN, NT, LE>;
     using Ix = IdxT<I32>;
     constexpr int NB = S::E / S::R0;
@@ -526,6 +532,34 @@ __device__ __forceinline__ void fft_tile_load(const TileArgs<T> &a, int64_t tile
             }
         }
     };
+    if constexpr (!std::is_same<LP, PlainLoad>::value) {
+        if (lp.in) {
+            // the tile's table entries first, then its elements: the two are
+            // dependent loads, so each kind issues as a whole
+            int at[S::E];
+            Ix base[NB];
+#pragma unroll
+            for (int e = 0; e < NB; ++e) {
+                int b, i;
+                bfly_pos<S::LOGB, LOGNR>(threadIdx.x + e * NT, a.seqfast_in, b, i);
+                const SeqPos<Ix> sp = seq_pos<Ix>(a, s0 + b);
+                base[e] = sp.in_base;
+#pragma unroll
+                for (int r = 0; r < S::R0; ++r) {
+                    const Ix gidx = Ix(i + r * NR) * in_gn + sp.j * in_gj;
+                    at[e * S::R0 + r] = sp.ok && gidx < nv ? ldg(lp.in, gidx) : -1;
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < NB; ++e)
+#pragma unroll
+                for (int r = 0; r < S::R0; ++r) {
+                    const int q = at[e * S::R0 + r];
+                    v[e * S::R0 + r] = q >= 0 ? ldg(a.x, Ix(base[e] + Ix(q))) : mk(T(0), T(0));
+                }
+            return;
+        }
+    }
     if (a.stream_out & 2)
         body([&](Ix k) { return ldg_stream(a.x, k); });
     else
@@ -555,9 +589,10 @@ __device__ __forceinline__ void tile_residual_sum(const TileArgs<T> &a, int64_t 
 }
 
 // Epilogue of a pass's store: none (plain stores), or an object whose
-// store<Ix, R>(idx, ok, u) takes over R elements u at offsets idx (those with
-// ok set) of the output's layout; it is called for a few elements at a time
-// so that it can load all of them before its first store.
+// store<Ix, R>(idx, row, ok, u) takes over R elements u at offsets idx (those
+// with ok set) of the output's layout, which are elements `row` of their columns;
+// it is called for a few elements at a time so that it can load all of them
+// before its first store.
 struct PlainStore {};
 constexpr int kEpilogueElems = 8;
 
@@ -636,15 +671,16 @@ __device__ __forceinline__ void fft_tile_store(const TileArgs<T> &a, int64_t til
             constexpr int C = RL < kEpilogueElems ? RL : kEpilogueElems;
 #pragma unroll
             for (int r0 = 0; r0 < RL; r0 += C) {
-                Ix idx[C];
+                Ix idx[C], row[C];
                 bool ok[C];
 #pragma unroll
                 for (int r = 0; r < C; ++r) {
                     const Ix n = Ix(i + (r0 + r) * NRL);
-                    ok[r] = n * out_gn + sp.j * out_gj < mv;
+                    row[r] = n * out_gn + sp.j * out_gj;
+                    ok[r] = row[r] < mv;
                     idx[r] = sp.out_base + n * out_ns;
                 }
-                ep.template store<Ix, C>(idx, ok, v + e * RL + r0);
+                ep.template store<Ix, C>(idx, row, ok, v + e * RL + r0);
             }
             continue;
         }
@@ -799,11 +835,11 @@ __device__ __forceinline__ void fft_tile_compute(const TileArgs<T> &a, int64_t t
 }
 
 template <typename T, int LOGN, int NT, bool CONV, bool I32 = false, int LE = -1,
-          typename EP = PlainStore>
+          typename EP = PlainStore, typename LP = PlainLoad>
 __device__ __forceinline__ void fft_pass_body(const TileArgs<T> &a, int64_t tile, cpx<T> *lds,
-                                              const EP &ep = EP()) {
+                                              const EP &ep = EP(), const LP &lp = LP()) {
     cpx<T> v[TileShape<T, LOGN, NT, LE>::E];
-    fft_tile_load<T, LOGN, NT, I32, LE>(a, tile, v);
+    fft_tile_load<T, LOGN, NT, I32, LE, LP>(a, tile, v, lp);
     fft_tile_compute<T, LOGN, NT, CONV, I32, LE, EP>(a, tile, v, lds, ep);
 }
 

@@ -303,9 +303,10 @@ int chunk_lanes(const Lanes *l);
 // stream, or NULL).
 int64_t chunk_columns(const Geometry &g, int64_t k, size_t esz, const Lanes *l);
 
-template <typename T>
-inline fm_status run_pipeline(const Geometry &g, const PipeIO &io, hipStream_t stream,
-                              const Lanes *lanes = nullptr) {
+// launch(pass, index, passes, stream) runs one pass of the transform.
+template <typename T, typename Launch>
+inline fm_status run_pipeline_with(const Geometry &g, const PipeIO &io, hipStream_t stream,
+                                   const Lanes *lanes, const Launch &launch) {
     const int64_t cc = chunk_columns(g, io.k, sizeof(cpx<T>), lanes);
     const int nl = cc < io.k ? chunk_lanes(lanes) : 1;
     const int64_t lane_bytes = (int64_t(1) << g.logL) * cc * int64_t(sizeof(cpx<T>));
@@ -325,7 +326,7 @@ inline fm_status run_pipeline(const Geometry &g, const PipeIO &io, hipStream_t s
         PassList<T> passes;
         fm_status st = build_pipeline<T>(g, sub, &passes);
         for (int p = 0; !st && p < passes.size(); ++p)
-            st = launch_tile<T>(passes[p].a, passes[p].conv, s);
+            st = launch(passes[p], p, passes.size(), s);
         if (st) return st;
     }
     if (nl > 1) {
@@ -333,6 +334,15 @@ inline fm_status run_pipeline(const Geometry &g, const PipeIO &io, hipStream_t s
         FM_CHECK_HIP(hipStreamWaitEvent(stream, lanes->join, 0));
     }
     return FM_SUCCESS;
+}
+
+template <typename T>
+inline fm_status run_pipeline(const Geometry &g, const PipeIO &io, hipStream_t stream,
+                              const Lanes *lanes = nullptr) {
+    return run_pipeline_with<T>(g, io, stream, lanes,
+                                [](const PassSpec<T> &p, int, int, hipStream_t s) {
+                                    return launch_tile<T>(p.a, p.conv, s);
+                                });
 }
 
 inline fm_status run_pipeline_any(const Geometry &g, const PipeIO &io, hipStream_t stream,

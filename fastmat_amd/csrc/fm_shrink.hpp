@@ -34,7 +34,8 @@ template <typename T> struct ShrinkStore {
     const ShrinkArgs<T> &s;
     T beta;
     template <typename Ix, int R>
-    __device__ __forceinline__ void store(const Ix *idx, const bool *ok, const cpx<T> *g) const {
+    __device__ __forceinline__ void store(const Ix *idx, const Ix *, const bool *ok,
+                                          const cpx<T> *g) const {
         // y, x and y_next may be one buffer: every load before the first store
         cpx<T> y[R], xo[R];
 #pragma unroll

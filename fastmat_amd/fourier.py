@@ -16,6 +16,7 @@ import ctypes
 import weakref
 
 import numpy as np
+import torch
 
 from . import _device as D
 from . import _lib
@@ -154,6 +155,43 @@ class Fourier(Matrix):
                   None if pre is None else _lib.ptr(pre), None if post is None else _lib.ptr(post),
                   _lib.ptr(X), n, _lib.ptr(Y), n, k, None if ws is None else _lib.ptr(ws),
                   need.value, D.stream())
+        return Y
+
+    def _select_ok(self, X):
+        """True when the passes over X can read and store selected elements: data
+        of the compute type, and a transform whose first and last passes are
+        plain ones of the lengths the selecting kernels have (a one-pass chirp
+        transform has one spectrum pass; four-step passes up to 2048 points)."""
+        if (D.np_dtype(X.dtype) != self.compute_dtype(X.dtype) or
+                D.promote(X.dtype, self._minType) != D.np_dtype(X.dtype)):
+            return False
+        n = self._order
+        if n & (n - 1) == 0:
+            return n <= 1 << 22
+        one_pass = 8192 if X.dtype == torch.complex64 else 4096
+        return one_pass < 2 * n - 1 <= 1 << 22
+
+    def _run_select(self, X, adjoint, pre, post, in_index, out_index, m):
+        """_run_diag that takes element in_index[i] of X's columns (zero where
+        negative) as element i of the transform's input, and stores element i of
+        its result as element out_index[i] of m (dropped where negative); see
+        _select_ok, and _diag_ok for pre and post.  Index tables are int32 device
+        vectors of the order's length, or None.  None when the block is beyond
+        the kernels' 32-bit offsets."""
+        h = self._plans.get(precision_of(X.dtype))
+        k, n = X.shape
+        Y = X.new_empty((k, m))
+        need = ctypes.c_int64()
+        _lib.call("fm_fourier_workspace_size", h, k, ctypes.byref(need))
+        ws = D.workspace(need.value)
+        try:
+            _lib.call("fm_fourier_apply_select", h, int(adjoint),
+                      *(None if t is None else _lib.ptr(t)
+                        for t in (pre, post, in_index, out_index)),
+                      _lib.ptr(X), n, _lib.ptr(Y), m, k, None if ws is None else _lib.ptr(ws),
+                      need.value, D.stream())
+        except NotImplementedError:
+            return None
         return Y
 
     def _apply_views(self, X, Y, adjoint):

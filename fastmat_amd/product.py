@@ -105,18 +105,80 @@ def _fourier_with_diags(factors, i, X, adjoint):
         return None
     F, flip = _as_fourier(factors[f])
     post = factors[f + 1] if f + 1 < len(factors) and type(factors[f + 1]) is Diag else None
-    if F is None or (pre is None and post is None) or not F._diag_ok(X):
-        return None
-    dt = D.np_dtype(X.dtype)
-    if not all(d is None or (D.promote(dt, d.dtype) == dt and D.promote(dt, d._minType) == dt)
-               for d in (pre, post)):
+    if F is None or (pre is None and post is None) or not _diags_ok(F, X, pre, post):
         return None
     # the transform conjugates its tables when it is an adjoint one; a Diag's
     # adjoint is its conjugate
     inverse = adjoint != flip
+    dt = D.np_dtype(X.dtype)
     Y = F._run_diag(X, inverse, None if pre is None else pre._table(dt, inverse != adjoint),
                     None if post is None else post._table(dt, inverse != adjoint))
     return Y, f + 1 + (post is not None)
+
+
+def _diags_ok(F, X, *diags):
+    """True when the Diag factors (or None) can run inside F's transform of X."""
+    dt = D.np_dtype(X.dtype)
+    return F._diag_ok(X) and all(
+        d is None or (D.promote(dt, d.dtype) == dt and D.promote(dt, d._minType) == dt)
+        for d in diags)
+
+
+def select_chain(M, X, adjoint, select_in, select_out, tables, m):
+    """M X or M^H X with the elements of X's columns and / or those of the result
+    (m of them) selected by the index tables that tables() returns
+    (Fourier._run_select; tables() is None where there are none), for a Fourier
+    matrix or a Product of one with a Diag on either or both sides of it; None
+    where the passes cannot do that.
+
+    The Diag factors run inside the passes where that holds without selection;
+    otherwise a Diag on a side that is not selected runs apart."""
+    if type(M) is Product:
+        factors = M._content if adjoint else M._content[::-1]
+        scalar = M._scalar != 1
+    else:
+        factors, scalar = (M,), False
+    if len(factors) > 3:
+        return None
+    pre = factors[0] if type(factors[0]) is Diag else None
+    f = int(pre is not None)
+    F, flip = _as_fourier(factors[f]) if f < len(factors) else (None, False)
+    post = factors[f + 1] if f + 1 < len(factors) and type(factors[f + 1]) is Diag else None
+    if F is None or f + 1 + (post is not None) != len(factors):
+        return None
+    t = D.input_type(X.dtype, M._minType, M.dtype, M._widenInputDatatype)
+    if X.dtype is not t:
+        X = X.to(t)
+    if type(M) is Product:
+        dt = D.promote(X.dtype, M.dtype)
+        if D.np_dtype(X.dtype) != dt:
+            X = X.to(D.torch_dtype(dt))
+    if pre is None:
+        # (the transform's own type rules: real data becomes complex)
+        X = X.to(D.torch_dtype(F.compute_dtype(
+            D.input_type(X.dtype, F._minType, F.dtype, F._widenInputDatatype))))
+    if not F._select_ok(X):
+        return None
+    inside = _diags_ok(F, X, pre, post)
+    if not inside and ((pre is not None and select_in) or (post is not None and select_out)):
+        return None
+    index = tables()
+    if index is None:
+        return None
+    if scalar:
+        X = M._prep(X, adjoint and np.iscomplexobj(M._scalar))
+    inverse = adjoint != flip
+    dt = D.np_dtype(X.dtype)
+    diags = [None if d is None or not inside else d._table(dt, inverse != adjoint)
+              for d in (pre, post)]
+    if pre is not None and not inside:
+        X = pre._apply(X, adjoint)
+        if not F._select_ok(X):
+            return None
+    Y = F._run_select(X, inverse, *diags, *index, m)
+    if Y is not None and post is not None and not inside:
+        Y = post._apply(Y, adjoint)
+    return Y
 
 
 def _as_fourier(f):

@@ -115,6 +115,18 @@ fm_status fm_fourier_apply_diag(const fm_fourier_plan *plan, int adjoint, const 
                                 const void *post, const void *x, int64_t ldx, void *y,
                                 int64_t ldy, int64_t k, void *workspace,
                                 int64_t workspace_bytes, void *stream);
+/* fm_fourier_apply_diag on selected elements of the columns (Partial.pyx:268-294
+ * around a Fourier matrix).  in_index[i] (order entries, device): element of the
+ * x column that is element i of the transform's input, negative for zero.
+ * out_index[i]: element of the y column that element i of the result is stored
+ * at, negative to drop it.  Either may be NULL (all elements in place).  pre and
+ * post: power-of-two orders only.  FM_ERR_NOT_IMPLEMENTED, before any launch, for
+ * one-pass chirp transforms, lengths above 2^22 and columns beyond 32-bit offsets. */
+fm_status fm_fourier_apply_select(const fm_fourier_plan *plan, int adjoint, const void *pre,
+                                  const void *post, const int32_t *in_index,
+                                  const int32_t *out_index, const void *x, int64_t ldx, void *y,
+                                  int64_t ldy, int64_t k, void *workspace,
+                                  int64_t workspace_bytes, void *stream);
 /* Mode-wise DFT along a strided axis (Kron mode application,
  * Kron.pyx:267-303): vectors v[i] = x[(o*N + i)*inner + j]; requires a
  * single-pass plan (N up to the LDS tile size). */
