@@ -114,8 +114,8 @@ _PROTOTYPES = {
                                 _vp, _vp, _vp, ctypes.c_double, _vp, _vp]),
     "fm_counter_advance": (_c_int, [_vp, _vp]),
     "fm_conv_shrink_workspace_size": (_c_int, [_vp, _c_i64, ctypes.POINTER(_c_i64)]),
-    "fm_conv_shrink_step": (_c_int, [_vp, _vp, _vp, _c_i64, ctypes.c_double, ctypes.c_double, _vp,
-                                     _vp, _vp, _vp, _vp, _vp, _c_i64, _vp]),
+    "fm_conv_shrink_run": (_c_int, [_vp, _vp, _vp, _c_i64, ctypes.c_double, ctypes.c_double, _vp,
+                                    _vp, _vp, _vp, _c_i64, _c_int, _vp, _c_i64, _vp]),
     "fm_lfsr_sequence": (_c_int, [ctypes.c_uint32, ctypes.c_uint32, _c_int,
                                   ctypes.POINTER(_c_i64), _vp, _vp, _c_i64]),
     "fm_lfsr_apply": (_c_int, [_c_int, _c_int, _c_i64, _vp, _vp, _vp, _c_i64, _vp, _c_i64, _c_i64,

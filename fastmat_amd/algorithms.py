@@ -153,7 +153,7 @@ class _Shrinkage(Algorithm):
         return w
 
     def _fused(self, wdt, k):
-        """(plan, workspace) of the one-call step (fm_conv_shrink_step), or
+        """(plan, workspace) of the fused steps (fm_conv_shrink_run), or
         None: a one-level Circulant or Toeplitz whose products have the
         iterate's dtype."""
         A = self.fmatA
@@ -169,21 +169,45 @@ class _Shrinkage(Algorithm):
             return None
         return h, D.workspace(need.value)
 
-    def _step(self, B, X, Y, Step, L, alpha, betas, counter, wdt, fused=None, keep_step=True):
+    def _run_fused(self, fused, B, X, Y, Step, L, alpha, betas, at, steps, flags):
+        """Steps at .. at + steps - 1 of a fused run (betas: all steps' momentum on
+        the host, or None; Step: None where the last one's is not needed)."""
+        h, ws = fused
+        _lib.call("fm_conv_shrink_run", h, _lib.ptr(Y), _lib.ptr(B), X.shape[0], float(L),
+                  float(alpha), _lib.ptr(X), None if Step is None else _lib.ptr(Step),
+                  _lib.ptr(Y) if self._momentum else None,
+                  None if betas is None else betas.ctypes.data + 8 * at, steps, flags,
+                  _lib.ptr(ws), ws.numel(), D.stream())
+
+    def _process_fused(self, fused, B, X, Y, Step, alpha, betas, steps, on_device):
+        """All steps by fm_conv_shrink_run.  A step leaves its next point's column
+        transform in the workspace for the step after it, unless a callback wrote
+        to the iterate in between.  Without callbacks a call runs 64 steps: few
+        enough that an interrupt is seen between calls."""
+        if self.cbStep is None and self.cbTrace is None:
+            for at in range(0, steps, 64):
+                n = min(64, steps - at)
+                last = at + n == steps
+                self._run_fused(fused, B, X, Y, Step if last else None, self.numL, alpha, betas,
+                                at, n, (1 if at else 0) | (0 if last else 2))
+            self.numStep = steps - 1
+            return
+        version = None
+        for self.numStep in range(steps):
+            same = version is not None and X._version == version
+            self._run_fused(fused, B, X, Y, Step, self.numL, alpha, betas, self.numStep, 1,
+                            (1 if same else 0) | (0 if self.numStep == steps - 1 else 2))
+            # (inference tensors do not count their versions)
+            version = None if X.is_inference() else X._version
+            self._expose(X, Step, on_device)
+            self.handleCallback(self.cbStep)
+            self.handleCallback(self.cbTrace)
+
+    def _step(self, B, X, Y, Step, L, alpha, betas, counter, wdt):
         """One iteration on the device: Y is the point the gradient is taken
-        at (X itself for ISTA).  The fused step writes Step only where
-        keep_step asks for it (nothing reads it between steps)."""
+        at (X itself for ISTA)."""
         A = self.fmatA
         k = X.shape[0]
-        if fused is not None:
-            h, ws = fused
-            _lib.call("fm_conv_shrink_step", h, _lib.ptr(Y), _lib.ptr(B), k, float(L),
-                      float(alpha), _lib.ptr(X), _lib.ptr(Step) if keep_step else None,
-                      _lib.ptr(Y) if self._momentum else None,
-                      _lib.ptr(betas) if betas is not None else None,
-                      _lib.ptr(counter) if counter is not None else None,
-                      _lib.ptr(ws), ws.numel(), D.stream())
-            return
         F = A._apply(Y, False)
         if D.np_dtype(F.dtype) != wdt:
             F = F.to(D.torch_dtype(wdt))
@@ -224,26 +248,43 @@ class _Shrinkage(Algorithm):
         X = D.empty(k, A.numCols, wdt).zero_()
         Y = X.clone() if self._momentum else X
         Step = torch.zeros_like(X)
-        betas = counter = None
+        steps = int(self.numMaxSteps)
+        betas = None
         if self._momentum:
             t, bl = 1.0, []
-            for _ in range(int(self.numMaxSteps)):
+            for _ in range(steps):
                 t_old = t
                 t = (1 + np.sqrt(1 + 4 * t ** 2)) / 2
                 bl.append((t_old - 1) / t)
-            betas = torch.tensor(bl, dtype=torch.float64, device=X.device)
-            # the step index, and the fused step's count of finished workgroups
-            counter = torch.zeros(2, dtype=torch.int64, device=X.device)
+            betas = np.array(bl, dtype=np.float64)
         fused = self._fused(wdt, k)
-        callbacks = self.cbStep is not None or self.cbTrace is not None
-        steps = int(self.numMaxSteps)
+        if fused is not None:
+            self._process_fused(fused, Bd, X, Y, Step, alpha, betas, steps, on_device)
+        else:
+            self._process_apart(Bd, X, Y, Step, alpha, betas, steps, wdt, on_device)
+        res = torch.where(X != 0, Step, X)
+        self._expose(X, Step, on_device)
+        if on_device:
+            self.arrResult = res.t()
+        else:
+            torch.cuda.synchronize()
+            self.arrResult = np.ascontiguousarray(res.cpu().numpy().T)
+        return self.arrResult
+
+    def _process_apart(self, Bd, X, Y, Step, alpha, betas, steps, wdt, on_device):
+        """All steps by separate applies; without callbacks the first runs eagerly
+        and one captured step is replayed for the rest."""
+        counter = None
+        if betas is not None:
+            betas = torch.tensor(betas, dtype=torch.float64, device=X.device)
+            counter = torch.zeros(1, dtype=torch.int64, device=X.device)
         self.numStep = 0
 
-        def step(keep_step=True):
-            self._step(Bd, X, Y, Step, self.numL, alpha, betas, counter, wdt, fused, keep_step)
+        def step():
+            self._step(Bd, X, Y, Step, self.numL, alpha, betas, counter, wdt)
 
-        step(callbacks or fused is None or steps == 1)
-        if callbacks:
+        step()
+        if self.cbStep is not None or self.cbTrace is not None:
             self._expose(X, Step, on_device)
             self.handleCallback(self.cbStep)
             self.handleCallback(self.cbTrace)
@@ -253,31 +294,17 @@ class _Shrinkage(Algorithm):
                 self.handleCallback(self.cbStep)
                 self.handleCallback(self.cbTrace)
         elif steps > 1:
-            # one step captured and replayed; a fused run ends with an eager
-            # step that writes Step
-            last = steps - 1 if fused is not None else steps
-            if last > 1:
-                graph = torch.cuda.CUDAGraph()
-                cur = torch.cuda.current_stream()
-                side = torch.cuda.Stream()
-                side.wait_stream(cur)
-                with torch.cuda.stream(side):
-                    with torch.cuda.graph(graph, stream=side):
-                        step(keep_step=fused is None)
-                cur.wait_stream(side)
-                for self.numStep in range(1, last):
-                    graph.replay()
-                del graph
-            for self.numStep in range(last, steps):
-                step()
-        res = torch.where(X != 0, Step, X)
-        self._expose(X, Step, on_device)
-        if on_device:
-            self.arrResult = res.t()
-        else:
-            torch.cuda.synchronize()
-            self.arrResult = np.ascontiguousarray(res.cpu().numpy().T)
-        return self.arrResult
+            graph = torch.cuda.CUDAGraph()
+            cur = torch.cuda.current_stream()
+            side = torch.cuda.Stream()
+            side.wait_stream(cur)
+            with torch.cuda.stream(side):
+                with torch.cuda.graph(graph, stream=side):
+                    step()
+            cur.wait_stream(side)
+            for self.numStep in range(1, steps):
+                graph.replay()
+            del graph
 
     def _expose(self, X, Step, on_device):
         """The reference's per-step attributes (arrX, arrStep), for callbacks

@@ -1,7 +1,7 @@
-// One ISTA / FISTA step on a 1-D convolution operator, with the residual and the
+// ISTA / FISTA steps on a 1-D convolution operator, with the residual and the
 // shrinkage inside the convolution's own passes.
 //
-// Replaces the operator applies and the numpy arithmetic of one step
+// Replaces the operator applies and the numpy arithmetic of the steps
 // (algorithms/ISTA.py:152-168, algorithms/FISTA.py:154-178):
 //     step   = y - L A^H (A y - b)
 //     x_new  = step * m / (m + alpha),   m = max(|step| - alpha, 0)
@@ -10,10 +10,15 @@
 // fused with the adjoint's column transform (inverse transform, residual, zero
 // beyond the rows, forward transform), so neither A y nor the residual is
 // written.  The adjoint's last pass holds A^H (A y - b) in registers and writes x
-// and y_next (and step where asked).  Per step and column of n = L elements that
-// is 14 blocks of reads and writes against 21 for applies, residual and shrinkage
-// apart, in 5 kernels instead of 9: 50 FISTA iterations on 2^18 x 8 complex64 take
-// 4.78 ms against 6.71 ms, bound by the latency of the 16 MB passes (11-23 us each).
+// and y_next (and step where asked); for a four-step it goes on with the next
+// step's column transform of y_next, whose columns are the same tile.  Per step and
+// column of n = L elements that is 13 blocks of reads and writes against 21 for
+// applies, residual and shrinkage apart, in 4 kernels instead of 9, launched one
+// after another from here (a replayed graph of one step took longer: its nodes
+// start 2 us apart, and it has to be captured and instantiated first).  50 FISTA
+// iterations on 2^18 x 8 complex64: 6.71 ms with nine kernels a step, 4.75 with a
+// replayed graph of five, 3.56 with these four (2 x 16.2, 16.8 and 21.8 us, the last
+// one 22.5 + 10.6 as two), bound by the latency of 16 MB passes.
 #pragma once
 
 #include "fm_fft_plan.hpp"
@@ -25,17 +30,16 @@ template <typename T> struct ShrinkArgs {
     cpx<T> *x;           // iterate, updated
     cpx<T> *step;        // NULL: not written
     cpx<T> *y_next;      // momentum point (may be y), or NULL
-    T L, alpha;
-    const double *beta_tab;  // momentum per step, or NULL (0)
-    int64_t *counter;        // [0] step index, [1] workgroups done (0 between launches)
+    T L, alpha, beta;    // beta: momentum of this step
 };
 
-template <typename T> struct ShrinkStore {
+// The shrinkage of a pass's elements: the store of a pass that ends with the
+// adjoint, or the middle of one that goes on with the next point's transform.
+template <typename T> struct Shrink {
     const ShrinkArgs<T> &s;
-    T beta;
+    // g: A^H (A y - b) on entry, the next point (0 outside the columns) on return
     template <typename Ix, int R>
-    __device__ __forceinline__ void store(const Ix *idx, const Ix *, const bool *ok,
-                                          const cpx<T> *g) const {
+    __device__ __forceinline__ void apply(const Ix *idx, const bool *ok, cpx<T> *g) const {
         // y, x and y_next may be one buffer: every load before the first store
         cpx<T> y[R], xo[R];
 #pragma unroll
@@ -48,47 +52,35 @@ template <typename T> struct ShrinkStore {
         }
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            if (!ok[r]) continue;
+            if (!ok[r]) {
+                g[r] = mk(T(0), T(0));
+                continue;
+            }
             const cpx<T> st = mk(y[r].x - s.L * g[r].x, y[r].y - s.L * g[r].y);
             const T m = fmax(T(hypot(st.x, st.y)) - s.alpha, T(0));
             const T f = m / (m + s.alpha);
             const cpx<T> xn = scale(st, f);
             if (s.step) stg(s.step, idx[r], st);
-            if (s.y_next)
-                stg(s.y_next, idx[r], xn + scale(xn - xo[r], beta));
+            g[r] = xn;
+            if (s.y_next) {
+                g[r] = xn + scale(xn - xo[r], s.beta);
+                stg(s.y_next, idx[r], g[r]);
+            }
             stg(s.x, idx[r], xn);
         }
     }
+    template <typename Ix, int R>
+    __device__ __forceinline__ void store(const Ix *idx, const Ix *, const bool *ok,
+                                          cpx<T> *g) const {
+        apply<Ix, R>(idx, ok, g);
+    }
 };
 
-// The adjoint's last pass with the shrinkage as its store.  The last workgroup to
-// finish moves the step counter on: by then every workgroup has read it.
-template <typename T, int LOGN, bool CONV, int LE, int NT>
-__global__ __launch_bounds__(NT) void fft_pass_shrink_kernel(const TileArgs<T> a,
-                                                             const ShrinkArgs<T> s) {
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    const ShrinkStore<T> ep{s, s.beta_tab ? T(s.beta_tab[s.counter[0]]) : T(0)};
-    fft_pass_body<T, LOGN, NT, CONV, true, LE, ShrinkStore<T>>(
-        a, xcd_remap(blockIdx.x, gridDim.x), reinterpret_cast<cpx<T> *>(smem_raw), ep);
-    if (s.beta_tab) {
-        // every thread's stores used beta, so the workgroup has read the counter
-        // by now; a relaxed count is enough (an agent-scope fence here would
-        // write the L2 back once per workgroup: 36 us a launch instead of 23)
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            const unsigned long long done =
-                __hip_atomic_fetch_add(reinterpret_cast<unsigned long long *>(s.counter + 1), 1ull,
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (done == gridDim.x - 1) {
-                s.counter[1] = 0;
-                s.counter[0] += 1;
-            }
-        }
-    }
-}
+// Where the shrinkage stands in a pass: after a column inverse (four-step), after a
+// one-pass convolution, or between a column inverse and a column transform.
+enum ShrinkPass { SHRINK_COLUMN, SHRINK_CONV, SHRINK_NEXT };
 
-// Launch of that pass: column pass (CONV = false) or one-pass convolution.
-template <typename T, bool CONV>
+template <typename T, int PASS>
 fm_status launch_shrink(const TileArgs<T> &a, const ShrinkArgs<T> &s, hipStream_t stream);
 
 // Lengths launch_shrink is compiled for.

@@ -2,8 +2,10 @@
 #include "fm_shrink_launch.hpp"
 
 namespace fm {
-template fm_status launch_shrink<float, false>(const TileArgs<float> &, const ShrinkArgs<float> &,
-                                          hipStream_t);
-template fm_status launch_shrink<float, true>(const TileArgs<float> &, const ShrinkArgs<float> &,
-                                         hipStream_t);
+#define FM_PASS(P) \
+    template fm_status launch_shrink<float, P>(const TileArgs<float> &, const ShrinkArgs<float> &, \
+                                               hipStream_t);
+FM_PASS(SHRINK_COLUMN)
+FM_PASS(SHRINK_CONV)
+FM_PASS(SHRINK_NEXT)
 }  // namespace fm

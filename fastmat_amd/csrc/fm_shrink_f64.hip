@@ -2,8 +2,10 @@
 #include "fm_shrink_launch.hpp"
 
 namespace fm {
-template fm_status launch_shrink<double, false>(const TileArgs<double> &, const ShrinkArgs<double> &,
-                                          hipStream_t);
-template fm_status launch_shrink<double, true>(const TileArgs<double> &, const ShrinkArgs<double> &,
-                                         hipStream_t);
+#define FM_PASS(P) \
+    template fm_status launch_shrink<double, P>(const TileArgs<double> &, const ShrinkArgs<double> &, \
+                                               hipStream_t);
+FM_PASS(SHRINK_COLUMN)
+FM_PASS(SHRINK_CONV)
+FM_PASS(SHRINK_NEXT)
 }  // namespace fm

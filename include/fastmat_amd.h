@@ -448,22 +448,24 @@ fm_status fm_shrink_step(int dtype, int64_t n, const void *y, const void *g, dou
                          const int64_t *step_counter, double beta, void *y_next,
                          void *stream);
 fm_status fm_counter_advance(int64_t *step_counter, void *stream);
-/* One whole ISTA / FISTA step on a one-level convolution plan A, every block
- * contiguous and in the plan's precision: with r = A y - b (rows x k) and
- * g = A^H r formed inside the convolution's passes,
+/* ISTA / FISTA steps on a one-level convolution plan A, every block contiguous and
+ * in the plan's precision: per step, with r = A y - b (rows x k) and g = A^H r
+ * formed inside the convolution's passes,
  *   step = y - L g,  x = step m / (m + alpha),  m = max(|step| - alpha, 0),
  *   y_next = x + beta (x - x_old).
- * x, step, y_next: cols x k; step may be NULL (not written), y_next NULL (no
- * momentum) or y, y may be x when y_next is NULL.  With beta_table, beta =
- * beta_table[counter[0]] and the step ends with counter[0] + 1; counter is two
- * device int64, the second 0.  Without, beta = 0 and counter is NULL.
+ * x, step, y_next: cols x k; step (of the last step; the others' are not written)
+ * may be NULL, y_next NULL (no momentum) or y, y may be x when y_next is NULL, and
+ * for more than one step the next point takes y's place.  betas: host array of
+ * `steps` values, or NULL for 0.  flags: 1 the workspace still holds the next
+ * point's transform that a call with flag 2 left (same y, not written since), 2
+ * leave it there.
  * FM_ERR_NOT_IMPLEMENTED (also from the workspace query) for plans without a
  * fused step: two-level plans, blocks of 4 GiB, lengths beyond 2^23. */
 fm_status fm_conv_shrink_workspace_size(const fm_conv_plan *plan, int64_t k, int64_t *bytes);
-fm_status fm_conv_shrink_step(const fm_conv_plan *plan, const void *y, const void *b, int64_t k,
-                              double L, double alpha, void *x, void *step, void *y_next,
-                              const double *beta_table, int64_t *counter, void *workspace,
-                              int64_t workspace_bytes, void *stream);
+fm_status fm_conv_shrink_run(const fm_conv_plan *plan, const void *y, const void *b, int64_t k,
+                             double L, double alpha, void *x, void *step, void *y_next,
+                             const double *betas, int64_t steps, int flags, void *workspace,
+                             int64_t workspace_bytes, void *stream);
 
 /* LFSRCirculant (LFSRCirculant.pyx:159-237): host-side register sequences.
  * Runs the generating register from `start` (masked to `order` bits) until
