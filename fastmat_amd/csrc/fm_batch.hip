@@ -1651,11 +1651,12 @@ extern "C" fm_status fm_batch_plan_destroy(fm_batch_plan *p) {
     if (p->gtab) (void)hipFree(p->gtab);
     if (p->stab) (void)hipFree(p->stab);
     if (p->res_part) (void)hipFree(p->res_part);
-    for (int q = 0; q < fm_batch_plan::kSide; ++q) {
-        if (p->side[q]) (void)hipStreamDestroy(p->side[q]);
-        if (p->join_ev[q]) (void)hipEventDestroy(p->join_ev[q]);
-    }
+    // the events before the streams they were recorded on
     if (p->fork_ev) (void)hipEventDestroy(p->fork_ev);
+    for (int q = 0; q < fm_batch_plan::kSide; ++q) {
+        if (p->join_ev[q]) (void)hipEventDestroy(p->join_ev[q]);
+        if (p->side[q]) (void)hipStreamDestroy(p->side[q]);
+    }
     delete p;
     return FM_SUCCESS;
 }

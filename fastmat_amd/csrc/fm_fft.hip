@@ -173,9 +173,10 @@ void lanes_create(Lanes *l) {
 }
 
 void lanes_destroy(Lanes *l) {
-    if (l->side) (void)hipStreamDestroy(l->side);
+    // the events before the stream they were recorded on
     if (l->fork) (void)hipEventDestroy(l->fork);
     if (l->join) (void)hipEventDestroy(l->join);
+    if (l->side) (void)hipStreamDestroy(l->side);
     *l = Lanes();
 }
 
