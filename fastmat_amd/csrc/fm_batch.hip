@@ -69,8 +69,22 @@ template <typename T> struct CorrDesc {
 // One persistent kernel per (length, conv, shape) class: grid-strided over the
 // class's (descriptor, tile) items.  SHAPE is SHAPE_WIDE or SHAPE_ROW (a batch
 // has no small launches).
+// Tile shapes of the batch's passes: those of the single-operator passes, except
+// that strided 512-point complex64 tiles hold 16 sequences in place of 8: with
+// non-temporal stores rows of 64 bytes are half cache lines written apart (column
+// passes of 2^18 x 32: 76-87 us, 61 with rows of 128 bytes).
+template <typename T, int LOGN, int SHAPE> struct BatchCfg {
+    static constexpr bool FULL = sizeof(T) == 4 && LOGN == 9 && SHAPE == SHAPE_WIDE;
+    static constexpr int LE = FULL ? 4 : PassCfg<T, LOGN, SHAPE>::LE;
+    static constexpr int NT = FULL ? 512 : PassCfg<T, LOGN, SHAPE>::NT;
+};
+template <typename T> static int batch_seqs(int logn, int shape) {
+    if (sizeof(T) == 4 && logn == 9 && shape == SHAPE_WIDE) return 16;
+    return pass_batch<T>(logn, shape);
+}
+
 template <typename T, int LOGN, bool CONV, int SHAPE, bool I32>
-__global__ __launch_bounds__((PassCfg<T, LOGN, SHAPE>::NT)) void batch_pass_kernel(
+__global__ __launch_bounds__((BatchCfg<T, LOGN, SHAPE>::NT)) void batch_pass_kernel(
     const BatchDesc<T> *__restrict__ descs, const int2 *__restrict__ items, int64_t nitems,
     int64_t out_shift, const T *__restrict__ out_mul) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -84,8 +98,8 @@ __global__ __launch_bounds__((PassCfg<T, LOGN, SHAPE>::NT)) void batch_pass_kern
             a.y = reinterpret_cast<cpx<T> *>(reinterpret_cast<char *>(a.y) + out_shift);
             if (out_mul) a.out_scale *= *out_mul;
         }
-        fft_pass_body<T, LOGN, PassCfg<T, LOGN, SHAPE>::NT, CONV, I32,
-                      PassCfg<T, LOGN, SHAPE>::LE>(a, w.y, lds);
+        fft_pass_body<T, LOGN, BatchCfg<T, LOGN, SHAPE>::NT, CONV, I32,
+                      BatchCfg<T, LOGN, SHAPE>::LE>(a, w.y, lds);
         __syncthreads();  // the next item reuses the LDS tile
     }
 }
@@ -328,7 +342,7 @@ static double pass_bytes(const TileArgs<double> &a, size_t esz) {
 template <typename T> static fm_status normalize_batch_pass(TileArgs<T> &a) {
     FM_REQUIRE(a.logN >= 0 && a.logN <= batch_max_log<T>(), FM_ERR_VALUE,
                "batched transform length 2^%d out of range", a.logN);
-    return normalize_pass(a, pass_batch<T>(a.logN, pick_shape(a, false)));
+    return normalize_pass(a, batch_seqs<T>(a.logN, pick_shape(a, false)));
 }
 
 // Normalise the descriptors, group work items into launches and upload.
@@ -449,7 +463,7 @@ static fm_status finalize(ProgBuilder<T> &b, Program &prog, int ncu_lanes_cap, h
 template <typename T, int LOGN, bool CONV, int SHAPE>
 static fm_status launch_pass_shape(const fm_batch_plan *p, const Program &d, const Launch &l,
                                    hipStream_t s, int64_t out_shift, const T *out_mul) {
-    const size_t lds = tile_lds_bytes<T>(LOGN, pass_batch<T>(LOGN, SHAPE));
+    const size_t lds = tile_lds_bytes<T>(LOGN, batch_seqs<T>(LOGN, SHAPE));
     static bool attr = false;
     if (!attr) {
         (void)hipFuncSetAttribute((const void *)batch_pass_kernel<T, LOGN, CONV, SHAPE, false>,
@@ -458,11 +472,16 @@ static fm_status launch_pass_shape(const fm_batch_plan *p, const Program &d, con
                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         attr = true;
     }
-    int64_t grid = int64_t(p->ncu) * p->grid_per_cu;
+    // a schedule's workgroups per CU count tiles of 64 KB: smaller tiles get as many
+    // more, or two per CU of a quarter of that leave a CU half empty (512-point row
+    // passes of 2^18 x 32: 111 us unscaled, 79 scaled)
+    constexpr int NT = BatchCfg<T, LOGN, SHAPE>::NT;
+    constexpr int64_t tile = (int64_t(NT) << BatchCfg<T, LOGN, SHAPE>::LE) * sizeof(cpx<T>);
+    constexpr int64_t share = tile < 65536 ? 65536 / tile : 1;
+    int64_t grid = int64_t(p->ncu) * p->grid_per_cu * share;
     if (grid > l.nitems) grid = l.nitems;
     ProfToken tok;
     prof_begin(s, &tok);
-    constexpr int NT = PassCfg<T, LOGN, SHAPE>::NT;
     if (l.idx32)
         hipLaunchKernelGGL((batch_pass_kernel<T, LOGN, CONV, SHAPE, true>), dim3(unsigned(grid)),
                            dim3(NT), lds, s, (const BatchDesc<T> *)d.descs, (const int2 *)l.items,
