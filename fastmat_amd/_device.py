@@ -159,21 +159,34 @@ def to_block(arr, required):
 
 
 # Row-major operands from this size on go through the library's transpose; torch's
-# strided copy costs the host less and is as fast below (2 MB complex128: 4.4 us).
+# strided copy costs the host 1.5 us less and is as fast below (2 MB complex128: 4.4 us).
 _TRANSPOSE_BYTES = 4 << 20
+
+
+def _transpose_bytes(esz, n, k):
+    """Size from which the library's transpose of n rows of k elements is the faster
+    one.  Measured, own / torch's copy in us:
+    4 and 8 bytes, rows of 8 elements on: 2^18 x 8 float32 6.4 / 7.4, 2^20 x 32 33 / 616,
+      2^18 x 32 float64 19 / 48; shorter rows only when large: 2^20 x 5 float32 8.8 / 7.7,
+      2^18 x 4 float64 6.1 / 5.9, but 2^22 x 2 float32 10 / 14, 2^20 x 4 float64 10 / 17;
+    16 bytes: 2^18 x 32 108 / 76 and 2^20 x 5 74 / 67, but 2^20 x 8 107 / 153;
+    1 byte: 2^22 x 8 38 / 28, but 2^18 x 16 6.8 / 7.6 and 2^22 x 32 121 / 600."""
+    if esz in (4, 8):
+        return _TRANSPOSE_BYTES * (1 if k >= 8 else 8)
+    pays = (k >= 6 and n >= 1 << 20) if esz == 16 else k >= 16
+    return _TRANSPOSE_BYTES * (1 if pays else 1 << 30)
 
 
 def contiguous_block(block):
     """The (k, n) view `block` as a contiguous tensor.  Columns of a large
     row-major (n, k) array on the device go through the library's transpose
-    (complex64 2^18 x 32: 26 us, torch's strided copy 63 us); small ones, other
-    layouts, lazily conjugated or negated tensors and tensor subclasses through
-    torch."""
+    (see _transpose_bytes); small ones, other layouts, lazily conjugated or
+    negated tensors and tensor subclasses through torch."""
     if block.is_contiguous():
         return block
     k, n = block.shape
     esz = block.element_size()
-    if k * n * esz >= _TRANSPOSE_BYTES and type(block) is torch.Tensor:
+    if k * n * esz >= _transpose_bytes(esz, n, k) and type(block) is torch.Tensor:
         s0, s1 = block.stride()
         if (s0 == 1 and s1 >= k and block.dtype in _T2NP and block.device == device() and
                 not block.is_conj() and not block.is_neg() and
