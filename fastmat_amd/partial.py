@@ -99,31 +99,38 @@ class Partial(Matrix):
     def _inverse(self, name, sel, dtype=torch.int64):
         """Row of the selection that lands on each row of the nested matrix's
         operand, -1 for none (the last one of equal indices, as numpy's
-        indexed assignment leaves it)."""
+        indexed assignment leaves it).  The table is complete before it is kept:
+        a later call may run on another stream.  None where it would have to be
+        made inside a stream capture, which does not run its kernels."""
         t = self._dev.get((name, dtype))
-        if t is None:
+        if t is None and not torch.cuda.is_current_stream_capturing():
             M = self._content[0]
             idx = self._idx(name, sel)
             t = torch.full((M.numRows if name == "r" else M.numCols,), -1, dtype=dtype,
                            device=idx.device)
             t.scatter_reduce_(0, idx, torch.arange(idx.numel(), dtype=dtype, device=idx.device),
                               "amax")
+            torch.cuda.current_stream(idx.device).synchronize()
             self._dev[name, dtype] = t
         return t
 
     def _distinct(self, name, sel):
         """True when no element is selected twice (counted on the device, once:
-        32 us on 2^18 elements, 190 in numpy)."""
+        32 us on 2^18 elements, 190 in numpy); False inside a stream capture
+        where it is not known yet."""
         d = self._dev.get("distinct" + name)
         if d is None:
-            hit = torch.count_nonzero(self._inverse(name, sel, torch.int32) >= 0)
-            d = self._dev["distinct" + name] = int(hit) == len(sel)
+            t = self._inverse(name, sel, torch.int32)
+            if t is None or torch.cuda.is_current_stream_capturing():
+                return False
+            d = self._dev["distinct" + name] = int(torch.count_nonzero(t >= 0)) == len(sel)
         return d
 
     def _selected(self, X, adjoint):
         """The product with both selections inside the passes of the nested
         Fourier matrix (select_chain), or None: other matrices, selections that
-        name an element twice for the result, and empty ones."""
+        name an element twice for the result, empty ones, and a capture before
+        the tables are there."""
         M = self._content[0]
         if type(M) not in (Product, Fourier, Hermitian) or X.shape[0] == 0:
             return None
@@ -140,8 +147,10 @@ class Partial(Matrix):
                     self._idx(name, sel)  # an index out of range is an error here
             if outs[1] is not None and not self._distinct(*outs):
                 return None
-            return [None if sel is None else self._inverse(name, sel, torch.int32)
+            made = [None if sel is None else self._inverse(name, sel, torch.int32)
                     for name, sel in (ins, outs)]
+            return made if all(s is None or t is not None
+                               for t, (_, s) in zip(made, (ins, outs))) else None
         return select_chain(M, X, adjoint, ins[1] is not None, outs[1] is not None, tables,
                             self.numCols if adjoint else self.numRows)
 
@@ -150,9 +159,13 @@ class Partial(Matrix):
         Y = D.empty(k, n_full, X.dtype)
         if n == 0:
             return Y.zero_()
-        _lib.call("fm_expand_rows", D.fm_type(X.dtype), n_full,
-                  _lib.ptr(self._inverse(name, sel)), _lib.ptr(X), n, _lib.ptr(Y), n_full, k,
-                  D.stream())
+        inverse = self._inverse(name, sel)
+        if inverse is None:  # (a capture that no call of this direction came before)
+            _lib.call("fm_scatter_rows", D.fm_type(X.dtype), n, _lib.ptr(self._idx(name, sel)),
+                      _lib.ptr(X), n, _lib.ptr(Y), n_full, n_full, k, D.stream())
+        else:
+            _lib.call("fm_expand_rows", D.fm_type(X.dtype), n_full, _lib.ptr(inverse),
+                      _lib.ptr(X), n, _lib.ptr(Y), n_full, k, D.stream())
         return Y
 
     def _gather(self, X, sel, name):
