@@ -182,8 +182,11 @@ class _Shrinkage(Algorithm):
     def _process_fused(self, fused, B, X, Y, Step, alpha, betas, steps, on_device):
         """All steps by fm_conv_shrink_run.  A step leaves its next point's column
         transform in the workspace for the step after it, unless a callback wrote
-        to the iterate in between.  Without callbacks a call runs 64 steps: few
-        enough that an interrupt is seen between calls."""
+        to the point in between.  Only ISTA's on the device can be written, the
+        iterate that the callback sees; its values tell, as no count of torch's
+        knows of a write through .data, DLPack or a raw address.  Without
+        callbacks a call runs 64 steps: few enough that an interrupt is seen
+        between calls."""
         if self.cbStep is None and self.cbTrace is None:
             for at in range(0, steps, 64):
                 n = min(64, steps - at)
@@ -192,13 +195,16 @@ class _Shrinkage(Algorithm):
                                 at, n, (1 if at else 0) | (0 if last else 2))
             self.numStep = steps - 1
             return
-        version = None
+        # (a one-pass plan keeps no transform)
+        seen = (torch.empty_like(X) if on_device and not self._momentum and
+                self.fmatA.plan_info(D.np_dtype(X.dtype))[3] > 1 else None)
         for self.numStep in range(steps):
-            same = version is not None and X._version == version
+            first, last = self.numStep == 0, self.numStep == steps - 1
+            same = not first and (seen is None or torch.equal(X, seen))
             self._run_fused(fused, B, X, Y, Step, self.numL, alpha, betas, self.numStep, 1,
-                            (1 if same else 0) | (0 if self.numStep == steps - 1 else 2))
-            # (inference tensors do not count their versions)
-            version = None if X.is_inference() else X._version
+                            (1 if same else 0) | (0 if last else 2))
+            if seen is not None and not last:
+                seen.copy_(X)
             self._expose(X, Step, on_device)
             self.handleCallback(self.cbStep)
             self.handleCallback(self.cbTrace)
