@@ -198,7 +198,12 @@ class _Shrinkage(Algorithm):
         # (a one-pass plan keeps no transform)
         seen = (torch.empty_like(X) if on_device and not self._momentum and
                 self.fmatA.plan_info(D.np_dtype(X.dtype))[3] > 1 else None)
+        A = self.fmatA
         for self.numStep in range(steps):
+            if self.fmatA is not A:  # a callback set another matrix
+                self._process_apart(B, X, Y, Step, alpha, betas, steps, D.np_dtype(X.dtype),
+                                    on_device, self.numStep)
+                return
             first, last = self.numStep == 0, self.numStep == steps - 1
             same = not first and (seen is None or torch.equal(X, seen))
             self._run_fused(fused, B, X, Y, Step, self.numL, alpha, betas, self.numStep, 1,
@@ -277,14 +282,14 @@ class _Shrinkage(Algorithm):
             self.arrResult = np.ascontiguousarray(res.cpu().numpy().T)
         return self.arrResult
 
-    def _process_apart(self, Bd, X, Y, Step, alpha, betas, steps, wdt, on_device):
-        """All steps by separate applies; without callbacks the first runs eagerly
-        and one captured step is replayed for the rest."""
+    def _process_apart(self, Bd, X, Y, Step, alpha, betas, steps, wdt, on_device, at=0):
+        """All steps from `at` on by separate applies; without callbacks the first
+        runs eagerly and one captured step is replayed for the rest."""
         counter = None
         if betas is not None:
             betas = torch.tensor(betas, dtype=torch.float64, device=X.device)
-            counter = torch.zeros(1, dtype=torch.int64, device=X.device)
-        self.numStep = 0
+            counter = torch.full((1,), at, dtype=torch.int64, device=X.device)
+        self.numStep = at
 
         def step():
             self._step(Bd, X, Y, Step, self.numL, alpha, betas, counter, wdt)
@@ -294,12 +299,12 @@ class _Shrinkage(Algorithm):
             self._expose(X, Step, on_device)
             self.handleCallback(self.cbStep)
             self.handleCallback(self.cbTrace)
-            for self.numStep in range(1, steps):
+            for self.numStep in range(at + 1, steps):
                 step()
                 self._expose(X, Step, on_device)
                 self.handleCallback(self.cbStep)
                 self.handleCallback(self.cbTrace)
-        elif steps > 1:
+        elif steps > at + 1:
             graph = torch.cuda.CUDAGraph()
             cur = torch.cuda.current_stream()
             side = torch.cuda.Stream()
@@ -308,7 +313,7 @@ class _Shrinkage(Algorithm):
                 with torch.cuda.graph(graph, stream=side):
                     step()
             cur.wait_stream(side)
-            for self.numStep in range(1, steps):
+            for self.numStep in range(at + 1, steps):
                 graph.replay()
             del graph
 

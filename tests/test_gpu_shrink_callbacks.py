@@ -65,3 +65,30 @@ def test_a_write_that_torch_does_not_count(kind, n, k, write):
     alg.process(b)
     ref = _ista_step(alg, A, b, seen["x"])
     assert (seen["next"] - ref).abs().max() <= 1e-4 * ref.abs().max()
+
+
+@pytest.mark.parametrize("other", ["circulant", "product"])
+@pytest.mark.parametrize("solver", ["ISTA", "FISTA"])
+@pytest.mark.parametrize("kind,n,k", [("c", 300, 2), ("c", 16384, 1)])
+def test_a_callback_that_sets_the_matrix(kind, n, k, solver, other):
+    """The step after takes the products of the matrix that is set, the one before
+    its own: a run that changes over to 3 A equals the steps by separate applies."""
+    import fastmat_amd as fm
+    from fastmat_amd import algorithms as fma
+    A, b = _problem(kind, n, k)
+    three = np.full(n, 3, np.complex64)
+    B = (fm.Circulant((3 * A._gen128).astype(np.complex64)) if other == "circulant"
+         else fm.Product(fm.Diag(three), A))
+    runs = []
+    for first in (A, fm.Product(A, fm.Eye(n))):
+        first._largestSV = 24.0
+
+        def callback(a):
+            if a.numStep == 2:
+                a.fmatA = B
+        print("set", solver, kind, n, k, other, type(first).__name__, flush=True)
+        alg = getattr(fma, solver)(first, numLambda=1e-3, numMaxSteps=6)
+        alg.cbStep = callback
+        runs.append(alg.process(b).clone())
+        assert alg.numStep == 5
+    assert (runs[0] - runs[1]).abs().max() <= 1e-4 * runs[1].abs().max()
