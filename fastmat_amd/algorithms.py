@@ -259,7 +259,7 @@ class _Shrinkage(Algorithm):
         X = D.empty(k, A.numCols, wdt).zero_()
         Y = X.clone() if self._momentum else X
         Step = torch.zeros_like(X)
-        steps = int(self.numMaxSteps)
+        steps = max(1, int(self.numMaxSteps))
         betas = None
         if self._momentum:
             t, bl = 1.0, []

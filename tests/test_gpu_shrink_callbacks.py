@@ -92,3 +92,15 @@ def test_a_callback_that_sets_the_matrix(kind, n, k, solver, other):
         runs.append(alg.process(b).clone())
         assert alg.numStep == 5
     assert (runs[0] - runs[1]).abs().max() <= 1e-4 * runs[1].abs().max()
+
+
+@pytest.mark.parametrize("solver", ["ISTA", "FISTA"])
+def test_less_than_one_step(solver):
+    """0.5 steps, which the check lets through, are one."""
+    import torch
+
+    from fastmat_amd import algorithms as fma
+    A, b = _problem("c", 300, 2)
+    runs = [getattr(fma, solver)(A, numLambda=1e-3, numMaxSteps=s) for s in (0.5, 1)]
+    x, ref = (alg.process(b) for alg in runs)
+    assert torch.equal(x, ref) and runs[0].numStep == 0
