@@ -35,6 +35,14 @@ class _PlanCache:
         self._destroy = destroy
         self._plans = {}
 
+    def __getstate__(self):
+        # (a weak reference does not go through pickle; an owner is being pickled
+        # with its cache, so the method is one of an object that comes along)
+        return dict(vars(self), _create=self._create())
+
+    def __setstate__(self, state):
+        vars(self).update(state, _create=weakref.WeakMethod(state["_create"]))
+
     def get(self, prec):
         h = self._plans.get(prec)
         if h is None:
