@@ -1,6 +1,7 @@
 """Diag: diagonal matrix (fastmat/Diag.pyx), GPU-backed element-wise kernel.
 Backward multiplies by conj(d) (Diag.pyx:159-167)."""
 import numpy as np
+import torch
 
 from . import _device as D
 from . import _lib
@@ -43,12 +44,17 @@ class Diag(Matrix):
         return t
 
     def _table(self, dt, conj):
-        """The diagonal on the device in the complex type dt, or its conjugate."""
+        """The diagonal on the device in the complex type dt, or its conjugate (a
+        table of its own, complete before it is kept; None where it would have to
+        be made inside a stream capture, which does not run its kernel)."""
+        d = self._d(dt)
         if not conj or self._vecD.dtype.kind != "c":
-            return self._d(dt)
+            return d
         t = self._dev.get((dt, "conj"))
-        if t is None:
-            t = self._dev[dt, "conj"] = D.as_tensor(self._vecD.conj(), dt)
+        if t is None and not torch.cuda.is_current_stream_capturing():
+            t = d.conj_physical()
+            torch.cuda.current_stream(d.device).synchronize()
+            self._dev[dt, "conj"] = t
         return t
 
     def _run(self, X, conj_d):

@@ -110,10 +110,19 @@ def _fourier_with_diags(factors, i, X, adjoint):
     # the transform conjugates its tables when it is an adjoint one; a Diag's
     # adjoint is its conjugate
     inverse = adjoint != flip
-    dt = D.np_dtype(X.dtype)
-    Y = F._run_diag(X, inverse, None if pre is None else pre._table(dt, inverse != adjoint),
-                    None if post is None else post._table(dt, inverse != adjoint))
-    return Y, f + 1 + (post is not None)
+    tables = _diag_tables(D.np_dtype(X.dtype), inverse != adjoint, pre, post)
+    if tables is None:
+        return None
+    return F._run_diag(X, inverse, *tables), f + 1 + (post is not None)
+
+
+def _diag_tables(dt, conj, *diags):
+    """Tables of the Diag factors (None for None), or None where one is missing
+    (Diag._table): the factors then run apart."""
+    tables = [None if d is None else d._table(dt, conj) for d in diags]
+    if any(t is None and d is not None for t, d in zip(tables, diags)):
+        return None
+    return tables
 
 
 def _diags_ok(F, X, *diags):
@@ -162,15 +171,14 @@ def select_chain(M, X, adjoint, select_in, select_out, tables, m):
     inside = _diags_ok(F, X, pre, post)
     if not inside and ((pre is not None and select_in) or (post is not None and select_out)):
         return None
-    index = tables()
+    inverse = adjoint != flip
+    diags = _diag_tables(D.np_dtype(X.dtype), inverse != adjoint,
+                         *((pre, post) if inside else (None, None)))
+    index = None if diags is None else tables()
     if index is None:
         return None
     if scalar:
         X = M._prep(X, adjoint and np.iscomplexobj(M._scalar))
-    inverse = adjoint != flip
-    dt = D.np_dtype(X.dtype)
-    diags = [None if d is None or not inside else d._table(dt, inverse != adjoint)
-              for d in (pre, post)]
     if pre is not None and not inside:
         X = pre._apply(X, adjoint)
         if not F._select_ok(X):

@@ -97,3 +97,40 @@ def test_capture_after_the_other_direction(name, both, adjoint):
         g.replay()
         torch.cuda.synchronize()
         _close(y, ref, dtype)
+
+
+@pytest.mark.parametrize("adjoint", [False, True])
+@pytest.mark.parametrize("selected", [False, True])
+def test_capture_of_a_product_after_the_other_direction(selected, adjoint):
+    """F^H D F with a complex D: one direction multiplies by D, the other by its
+    conjugate, a table of its own inside the passes."""
+    import torch
+
+    import fastmat_amd as fm
+    n, k = 1 << 14, 3
+    rng = np.random.default_rng(n)
+    d = (rng.standard_normal(n) + 1j * rng.standard_normal(n)).astype(np.complex64)
+    F = fm.Fourier(n)
+
+    def make():
+        M = fm.Product(F.H, fm.Diag(d), F)
+        return fm.Partial(M, rows=np.arange(0, n, 3)) if selected else M
+    P = make()
+    run, warm = (P.backward, P.forward) if adjoint else (P.forward, P.backward)
+    size, warm_size = (P.numRows, P.numCols) if adjoint else (P.numCols, P.numRows)
+    x = _data(size, k, np.complex64, 7)
+    warm(_data(warm_size, k, np.complex64, 6))
+    torch.cuda.synchronize()
+    print("capture product", selected, adjoint, flush=True)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        y = run(x)
+    Q = make()
+    _close(run(x), (Q.backward if adjoint else Q.forward)(x), np.complex64)
+    for seed in (8, 9, 10):
+        x.copy_(_data(size, k, np.complex64, seed))
+        ref = run(x)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        _close(y, ref, np.complex64)
