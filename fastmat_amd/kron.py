@@ -62,6 +62,9 @@ class Kron(Matrix):
         k = X.shape[0]
         dims = self._dims
         fused = _fused_tail(self._content, X.dtype)
+        # (a capture without the transposed table: the two modes apart)
+        A_d = self._content[-1]._device_f32(transposed=adjoint) if fused else None
+        fused = A_d is not None
         last = len(self._content) - (2 if fused else 0)
         for m, f in enumerate(self._content[:last]):
             outer = k * int(np.prod(dims[:m], dtype=np.int64))
@@ -75,8 +78,7 @@ class Kron(Matrix):
             Y = torch.empty_like(Xc)
             outer = k * int(np.prod(dims[:-2], dtype=np.int64))
             _lib.call("fm_kron_pair_apply", C.plan_handle(np.complex64), int(adjoint),
-                      _lib.ptr(A._device_f32(transposed=adjoint)), A.numRows, _lib.ptr(Xc),
-                      _lib.ptr(Y), outer, D.stream())
+                      _lib.ptr(A_d), A.numRows, _lib.ptr(Xc), _lib.ptr(Y), outer, D.stream())
             X = Y
         return X
 

@@ -356,15 +356,21 @@ class Matrix:
                 D.np_dtype(dtype) in (np.dtype(np.float32), np.dtype(np.complex64)))
 
     def _device_f32(self, transposed=False):
-        """The float32 array on the device, contiguous row-major (or its
-        transpose), cached."""
-        key = "f32T" if transposed else "f32"
-        A_d = self._dev.get(key)
+        """The float32 array on the device, contiguous row-major, cached; or its
+        transpose (complete before it is kept; None where it would have to be made
+        inside a stream capture, which does not run its kernel)."""
+        A_d = self._dev.get("f32")
         if A_d is None:
-            A = np.asarray(self._array, dtype=np.float32)
-            A_d = self._dev[key] = D.as_tensor(np.ascontiguousarray(A.T if transposed else A),
-                                               np.float32)
-        return A_d
+            A_d = self._dev["f32"] = D.as_tensor(np.asarray(self._array, dtype=np.float32),
+                                                 np.float32)
+        if not transposed:
+            return A_d
+        T_d = self._dev.get("f32T")
+        if T_d is None and not torch.cuda.is_current_stream_capturing():
+            T_d = A_d.t().contiguous()
+            torch.cuda.current_stream(A_d.device).synchronize()
+            self._dev["f32T"] = T_d
+        return T_d
 
     def _apply_strided(self, X, adjoint, outer, inner):
         A_d = self._device_f32()

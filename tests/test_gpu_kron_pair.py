@@ -37,3 +37,30 @@ def test_kron_pair_shapes(n, m, f, k):
     ref = fast64.kron_apply([lambda v: fast64.fourier(v, adjoint=True),
                              lambda v: C.conj().T @ v, lambda v: A64.T @ v], (f, n, m), x)
     assert accept.max_rel_error(K.backward(x), ref) < 1e-5
+
+
+@pytest.mark.parametrize("adjoint", [False, True])
+def test_capture_after_the_other_direction(adjoint):
+    """The pair takes the dense factor as it is or transposed, a table each: a capture
+    of one direction after a warm-up of the other alone equals the eager call (the
+    single precision bar, as the factors may run apart inside the capture)."""
+    import torch
+
+    import fastmat_amd as fm
+    rng = np.random.default_rng(5)
+    c = (rng.standard_normal(64) + 1j * rng.standard_normal(64)).astype(np.complex64)
+    K = fm.Kron(fm.Circulant(c), fm.Matrix(rng.standard_normal((96, 96)).astype(np.float32)))
+    x = torch.randn((3, 64 * 96), device="cuda", dtype=torch.complex64).t()
+    run, warm = (K.backward, K.forward) if adjoint else (K.forward, K.backward)
+    warm(x)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        y = run(x)
+    for _ in range(3):
+        x.copy_(torch.randn_like(x))
+        ref = run(x)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert (y - ref).abs().max() <= 1e-5 * ref.abs().max()
