@@ -49,29 +49,33 @@ template <typename T> struct ElemOps<cpx<T>> {
 // loads are all in flight together, and no element needs a division to find its
 // row (a flat grid-stride loop over n k elements did: 64-bit, ~40 instructions).
 constexpr int kElemCols = 8;
+// Workgroups per grid dimension: a dimension of a launch has less than 2^32
+// threads (and y at most 65535 workgroups); the kernels stride over the rest.
+constexpr int64_t kElemGridX = int64_t(1) << 22;
 static inline dim3 row_grid(int64_t n, int64_t k, unsigned *threads) {
     *threads = n >= 256 ? 256u : unsigned(ceil_div(n, 64) * 64);
-    const int64_t gy = ceil_div(k, kElemCols);
-    return dim3(unsigned(ceil_div(n, *threads)), unsigned(gy < 65535 ? gy : 65535));
+    const int64_t gx = ceil_div(n, *threads), gy = ceil_div(k, kElemCols);
+    return dim3(unsigned(std::min(gx, kElemGridX)), unsigned(std::min<int64_t>(gy, 65535)));
 }
 
-// f(first column, columns) for this thread's column groups, with a full group's
-// count as a constant.
-template <typename F> __device__ __forceinline__ void each_group(int64_t k, F f) {
-    for (int64_t j = blockIdx.y * int64_t(kElemCols); j < k; j += int64_t(gridDim.y) * kElemCols) {
-        if (j + kElemCols <= k) f(j, kElemCols);
-        else f(j, int(k - j));
-    }
+// f(row, first column, columns) for this thread's rows and column groups, with a
+// full group's count as a constant.
+template <typename F> __device__ __forceinline__ void each_group(int64_t n, int64_t k, F f) {
+    for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n;
+         i += int64_t(gridDim.x) * blockDim.x)
+        for (int64_t j = blockIdx.y * int64_t(kElemCols); j < k;
+             j += int64_t(gridDim.y) * kElemCols) {
+            if (j + kElemCols <= k) f(i, j, kElemCols);
+            else f(i, j, int(k - j));
+        }
 }
 
 // y[i, j] = x[i, j] * d[i] (or conj(d[i])), column-major n x k
 template <typename S>
 __global__ void diag_kernel(const S *__restrict__ d, const S *__restrict__ x, int64_t ldx,
                             S *__restrict__ y, int64_t ldy, int64_t n, int64_t k, int conj_d) {
-    const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-    if (i >= n) return;
-    const S di = d[i];
-    each_group(k, [&](int64_t j0, int cols) {
+    each_group(n, k, [&](int64_t i, int64_t j0, int cols) {
+        const S di = d[i];
         S v[kElemCols];
 #pragma unroll
         for (int c = 0; c < kElemCols; ++c)
@@ -94,29 +98,30 @@ template <typename S, bool EXPAND>
 __global__ __launch_bounds__(256) void gather_kernel(const int64_t *__restrict__ idx,
                                                      const S *__restrict__ x, int64_t ldx,
                                                      S *__restrict__ y, int64_t ldy, int64_t n_out,
-                                                     unsigned row_tiles) {
-    const unsigned tile = unsigned(xcd_remap(blockIdx.x, gridDim.x));
-    const unsigned col = tile / row_tiles;
-    const int64_t i0 = (tile - col * row_tiles) * int64_t(256 * kGatherRows) + threadIdx.x;
-    const S *xc = x + int64_t(col) * ldx;
-    S *yc = y + int64_t(col) * ldy;
-    int64_t r[kGatherRows];
+                                                     int64_t row_tiles, int64_t tiles) {
+    for (int64_t tile = xcd_remap(blockIdx.x, gridDim.x); tile < tiles; tile += gridDim.x) {
+        // (tile indices below 2^32, all but a few, divide as such)
+        const int64_t col = tile >> 32 ? tile / row_tiles : unsigned(tile) / unsigned(row_tiles);
+        const int64_t i0 = (tile - col * row_tiles) * int64_t(256 * kGatherRows) + threadIdx.x;
+        const S *xc = x + col * ldx;
+        S *yc = y + col * ldy;
+        int64_t r[kGatherRows];
 #pragma unroll
-    for (int e = 0; e < kGatherRows; ++e) r[e] = i0 + e * 256 < n_out ? idx[i0 + e * 256] : -1;
-    S v[kGatherRows] = {};
+        for (int e = 0; e < kGatherRows; ++e)
+            r[e] = i0 + e * 256 < n_out ? idx[i0 + e * 256] : -1;
+        S v[kGatherRows] = {};
 #pragma unroll
-    for (int e = 0; e < kGatherRows; ++e)
-        if (r[e] >= 0) v[e] = xc[r[e]];
+        for (int e = 0; e < kGatherRows; ++e)
+            if (r[e] >= 0) v[e] = xc[r[e]];
 #pragma unroll
-    for (int e = 0; e < kGatherRows; ++e)
-        if (EXPAND ? i0 + e * 256 < n_out : r[e] >= 0) yc[i0 + e * 256] = v[e];
+        for (int e = 0; e < kGatherRows; ++e)
+            if (EXPAND ? i0 + e * 256 < n_out : r[e] >= 0) yc[i0 + e * 256] = v[e];
+    }
 }
 
 template <typename S>
 __global__ void zero_kernel(S *__restrict__ y, int64_t ldy, int64_t n, int64_t k) {
-    const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-    if (i >= n) return;
-    each_group(k, [&](int64_t j0, int cols) {
+    each_group(n, k, [&](int64_t i, int64_t j0, int cols) {
 #pragma unroll
         for (int c = 0; c < kElemCols; ++c)
             if (c < cols) y[(j0 + c) * ldy + i] = S{};
@@ -127,10 +132,8 @@ template <typename S>
 __global__ void scatter_kernel(const int64_t *__restrict__ idx, const S *__restrict__ x,
                                int64_t ldx, S *__restrict__ y, int64_t ldy, int64_t n_in,
                                int64_t k) {
-    const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-    if (i >= n_in) return;
-    const int64_t r = idx[i];
-    each_group(k, [&](int64_t j0, int cols) {
+    each_group(n_in, k, [&](int64_t i, int64_t j0, int cols) {
+        const int64_t r = idx[i];
         S v[kElemCols];
 #pragma unroll
         for (int c = 0; c < kElemCols; ++c)
@@ -144,9 +147,7 @@ __global__ void scatter_kernel(const int64_t *__restrict__ idx, const S *__restr
 template <typename S>
 __global__ void axpby_kernel(S alpha, const S *x, int64_t ldx, int conj_x, S beta, int use_beta,
                              S *y, int64_t ldy, int64_t n, int64_t k) {
-    const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-    if (i >= n) return;
-    each_group(k, [&](int64_t j0, int cols) {
+    each_group(n, k, [&](int64_t i, int64_t j0, int cols) {
         S v[kElemCols], w[kElemCols];
 #pragma unroll
         for (int c = 0; c < kElemCols; ++c)
@@ -263,15 +264,10 @@ static fm_status gather_any(int64_t n_out, const int64_t *idx, const void *x, in
                           int64_t ldy, int64_t k, hipStream_t s) {
     ProfToken tok;
     prof_begin(s, &tok);
-    const int64_t row_tiles = ceil_div(n_out, 256 * kGatherRows);
-    // (the kernel's tile index is 32 bits wide: more columns in further launches)
-    const int64_t cols = std::max<int64_t>(1, ((int64_t(1) << 31) - 1) / row_tiles);
-    for (int64_t j = 0; j < k; j += cols) {
-        const int64_t kc = std::min(cols, k - j);
-        hipLaunchKernelGGL((gather_kernel<S, EXPAND>), dim3(unsigned(row_tiles * kc)), dim3(256), 0,
-                           s, idx, (const S *)x + j * ldx, ldx, (S *)y + j * ldy, ldy, n_out,
-                           unsigned(row_tiles));
-    }
+    const int64_t row_tiles = ceil_div(n_out, 256 * kGatherRows), tiles = row_tiles * k;
+    hipLaunchKernelGGL((gather_kernel<S, EXPAND>), dim3(unsigned(std::min(tiles, kElemGridX))),
+                       dim3(256), 0, s, idx, (const S *)x, ldx, (S *)y, ldy, n_out, row_tiles,
+                       tiles);
     FM_CHECK_LAUNCH();
     prof_elem(s, &tok, EXPAND ? "expand_kernel" : "gather_kernel", sizeof(S),
               2.0 * double(n_out) * double(k) * sizeof(S) + 8.0 * double(n_out));
