@@ -137,6 +137,7 @@ extern "C" fm_status fm_conv_shrink_run(const fm_conv_plan *p, const void *y, co
     if (st) return st;
     FM_REQUIRE(y && b && x && workspace, FM_ERR_VALUE, "NULL data pointer");
     FM_REQUIRE(steps >= 1, FM_ERR_VALUE, "at least one step expected");
+    FM_REQUIRE(alpha > 0.0, FM_ERR_VALUE, "shrinkage threshold must be positive");
     FM_REQUIRE(steps == 1 || y == (y_next ? y_next : x), FM_ERR_VALUE,
                "several steps need the next point in place of the point");
     FM_REQUIRE(workspace_bytes >= need, FM_ERR_VALUE,
