@@ -207,13 +207,20 @@ static fm_status transpose_launch(int64_t n, int64_t k, const void *src, int64_t
                                   int64_t ldd, hipStream_t s) {
     constexpr int LOGT = sizeof(S) == 16 ? 11 : 12;
     constexpr int TR = 1 << (LOGT - LOGC);
-    const int64_t gx = ceil_div(n, TR), gy = ceil_div(k, int64_t(1) << LOGC);
-    FM_REQUIRE(gx < (int64_t(1) << 31) && gy <= 65535, FM_ERR_VALUE,
-               "transpose of %lld x %lld is too large for one launch", (long long)n, (long long)k);
+    constexpr int TC = 1 << LOGC;
     ProfToken tok;
     prof_begin(s, &tok);
-    hipLaunchKernelGGL((transpose_kernel<S, LOGT, LOGC>), dim3(unsigned(gx), unsigned(gy)),
-                       dim3(256), 0, s, (const S *)src, lds_, (S *)dst, ldd, n, k);
+    // (a launch for what one grid does not take: loops in the kernel would hold its
+    // addresses in registers, 256 of them in place of 55)
+    constexpr int64_t rows = kElemGridX * TR, cols = 65535 * int64_t(TC);
+    for (int64_t i = 0; i < n; i += rows)
+        for (int64_t c = 0; c < k; c += cols) {
+            const int64_t nn = std::min(n - i, rows), kk = std::min(k - c, cols);
+            hipLaunchKernelGGL((transpose_kernel<S, LOGT, LOGC>),
+                               dim3(unsigned(ceil_div(nn, TR)), unsigned(ceil_div(kk, TC))),
+                               dim3(256), 0, s, (const S *)src + i * lds_ + c, lds_,
+                               (S *)dst + c * ldd + i, ldd, nn, kk);
+        }
     FM_CHECK_LAUNCH();
     prof_elem(s, &tok, "transpose_kernel", sizeof(S), 2.0 * double(n) * double(k) * sizeof(S));
     return FM_SUCCESS;
