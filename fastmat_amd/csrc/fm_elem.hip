@@ -11,6 +11,7 @@
 // reference's C loops.  All kernels work on n x k blocks of column-major data and
 // stream HBM once.
 #include <algorithm>
+#include <type_traits>
 
 #include "fm_common.hpp"
 
@@ -44,126 +45,166 @@ template <typename T> struct ElemOps<cpx<T>> {
     __host__ static cpx<T> from(const double *v) { return mk(T(v[0]), T(v[1])); }
 };
 
-// Launch shape of the row-wise kernels: a thread works on one row of a few
-// columns, so that a row's index or diagonal entry is read once for them, their
-// loads are all in flight together, and no element needs a division to find its
-// row (a flat grid-stride loop over n k elements did: 64-bit, ~40 instructions).
-constexpr int kElemCols = 8;
-// Workgroups per grid dimension: a dimension of a launch has less than 2^32
-// threads (and y at most 65535 workgroups); the kernels stride over the rest.
-constexpr int64_t kElemGridX = int64_t(1) << 22;
-static inline dim3 row_grid(int64_t n, int64_t k, unsigned *threads) {
-    *threads = n >= 256 ? 256u : unsigned(ceil_div(n, 64) * 64);
-    const int64_t gx = ceil_div(n, *threads), gy = ceil_div(k, kElemCols);
-    return dim3(unsigned(std::min(gx, kElemGridX)), unsigned(std::min<int64_t>(gy, 65535)));
+// Row-wise kernels: the n k elements of a launch in order, E of them a thread, 256
+// apart, so that a wave's accesses are contiguous, a thread's loads are all in flight
+// together and no lane idles whatever n and k are.  The column of element t is
+// floor(t / n), a multiplication by n's reciprocal.  Bound by HBM, and by the launch
+// below some 8 MB.  Measured in us against a thread per row of eight columns, which
+// leaves most lanes without a row below 64 rows and most columns empty below eight
+// (and a gather by tiles of 1024 rows of one column), and against a flat loop with a
+// 64-bit division per element:
+//   Diag    float32     4 x 2^20    61 /  8.5 ->   6.5     2^24 x 1    211 /  34 ->  32
+//           complex64  10^6 x 64   208 /  234 -> 194     2^20 x 16    62 /  44 ->  46
+//           complex128  4 x 2^20    74 /   21 ->  20     2^18 x 32    50 /  39 ->  38
+//   gather  float32     4 x 2^20   742 /  9.0 ->   7.2   10^6 x 64   404 / 917 -> 404
+//           complex64   4 x 2^20   738 / 13.5 ->  12.4    2^18 x 32   48 /  73 ->  46
+//           complex128  4 x 2^20   925 /   20 ->  20     2^18 x 32    96 / 108 ->  75
+// Slower than that loop: Diag on 3 x 5 10^7 int8 190 (175) and int16 247 (205), a third
+// of 2^20 x 16 float32 rows in order 20.7 (16.9).
+constexpr int kElemThreads = 256;
+struct Rows {
+    uint32_t total, n, mul, shift;
+    // column of element t < 2^31: for s = ceil(log2 n) and m = 2^32 (2^s / n - 1)
+    // rounded up, floor((t + floor(t m / 2^32)) / 2^s) = floor(t / n) (Granlund and
+    // Montgomery, "Division by invariant integers using multiplication")
+    __device__ __forceinline__ uint32_t column(uint32_t t) const {
+        return (__umulhi(t, mul) + t) >> shift;
+    }
+};
+
+// f(row, column) of this thread's elements e, where there is one.
+template <int E, typename F>
+__device__ __forceinline__ void each_element(const Rows &r, int64_t block, F f) {
+    const uint32_t t0 = uint32_t(block) * (kElemThreads * E) + threadIdx.x;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const uint32_t t = t0 + e * kElemThreads, j = r.column(t);
+        if (t < r.total) f(e, t - j * r.n, j);
+    }
 }
 
-// f(row, first column, columns) for this thread's rows and column groups, with a
-// full group's count as a constant.
-template <typename F> __device__ __forceinline__ void each_group(int64_t n, int64_t k, F f) {
-    for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n;
-         i += int64_t(gridDim.x) * blockDim.x)
-        for (int64_t j = blockIdx.y * int64_t(kElemCols); j < k;
-             j += int64_t(gridDim.y) * kElemCols) {
-            if (j + kElemCols <= k) f(i, j, kElemCols);
-            else f(i, j, int(k - j));
+// Elements per thread: four of up to 8 bytes, from the size on where that leaves every
+// CU four workgroups.
+constexpr uint32_t kElemMany = 1u << 20;
+template <typename S> constexpr int elem_each() { return sizeof(S) <= 8 ? 4 : 1; }
+
+// Launches of a row-wise kernel on n x k elements, of at most 2^30 each (one as a
+// rule): launch(elements per thread, rows, grid, first row, first column).
+template <int E, typename F> static void launch_rows(int64_t n, int64_t k, F launch) {
+    constexpr int64_t part = int64_t(1) << 30;
+    const int64_t rows = std::min(n, part), cols = std::max<int64_t>(1, part / rows);
+    for (int64_t j = 0; j < k; j += cols)
+        for (int64_t i = 0; i < n; i += rows) {
+            const uint64_t nn = std::min(n - i, rows), kk = std::min(k - j, cols);
+            Rows r;
+            r.total = uint32_t(nn * kk);
+            r.n = uint32_t(nn);
+            r.shift = 0;
+            while ((uint64_t(1) << r.shift) < nn) ++r.shift;
+            r.mul = uint32_t((((uint64_t(1) << r.shift) - nn) << 32) / nn + 1);
+            if (r.total >= kElemMany)
+                launch(std::integral_constant<int, E>(), r,
+                       dim3(ceil_div(r.total, E * kElemThreads)), i, j);
+            else
+                launch(std::integral_constant<int, 1>(), r, dim3(ceil_div(r.total, kElemThreads)),
+                       i, j);
         }
 }
 
 // y[i, j] = x[i, j] * d[i] (or conj(d[i])), column-major n x k
-template <typename S>
-__global__ void diag_kernel(const S *__restrict__ d, const S *__restrict__ x, int64_t ldx,
-                            S *__restrict__ y, int64_t ldy, int64_t n, int64_t k, int conj_d) {
-    each_group(n, k, [&](int64_t i, int64_t j0, int cols) {
-        const S di = d[i];
-        S v[kElemCols];
-#pragma unroll
-        for (int c = 0; c < kElemCols; ++c)
-            if (c < cols) v[c] = x[(j0 + c) * ldx + i];
-#pragma unroll
-        for (int c = 0; c < kElemCols; ++c)
-            if (c < cols)
-                y[(j0 + c) * ldy + i] =
-                    conj_d ? ElemOps<S>::mulc(v[c], di) : ElemOps<S>::mul(v[c], di);
+template <typename S, int E>
+__global__ __launch_bounds__(kElemThreads) void diag_kernel(const Rows r, const S *__restrict__ d,
+                                                            const S *__restrict__ x, int64_t ldx,
+                                                            S *__restrict__ y, int64_t ldy,
+                                                            int conj_d) {
+    S v[E], w[E];
+    each_element<E>(r, blockIdx.x, [&](int e, uint32_t i, uint32_t j) {
+        v[e] = x[j * ldx + i];
+        w[e] = d[i];
+    });
+    each_element<E>(r, blockIdx.x, [&](int e, uint32_t i, uint32_t j) {
+        y[j * ldy + i] = conj_d ? ElemOps<S>::mulc(v[e], w[e]) : ElemOps<S>::mul(v[e], w[e]);
     });
 }
+
+// The kernels that only move elements take them as bytes of their size (a conditional
+// copy of a complex128 object goes through LDS, 13 us a launch for it).
+typedef uint32_t Bytes16 __attribute__((ext_vector_type(4)));
+#define FM_DISPATCH_SIZE(dtype, FN, ...)                                                \
+    switch (dtype) {                                                                  \
+    case FM_INT8: return FN<uint8_t>(__VA_ARGS__);                                    \
+    case FM_INT16: return FN<uint16_t>(__VA_ARGS__);                                  \
+    case FM_INT32:                                                                    \
+    case FM_FLOAT32: return FN<uint32_t>(__VA_ARGS__);                                \
+    case FM_INT64:                                                                    \
+    case FM_FLOAT64:                                                                  \
+    case FM_COMPLEX64: return FN<uint64_t>(__VA_ARGS__);                              \
+    case FM_COMPLEX128: return FN<Bytes16>(__VA_ARGS__);                              \
+    default: set_error("Unsupported type: %d", dtype); return FM_ERR_TYPE;            \
+    }
 
 // y[i, j] = x[idx[i], j]; rows with idx[i] < 0 are zero (EXPAND).  The reads of
-// one column hit its cache lines in any order, so a column's tiles run together
-// and on one XCD: its lines then come from HBM once, into one L2, not once per
-// XCD (70001 of 2^18 rows x 32 complex64: 36 us with columns spread over all
-// XCDs, 39 us with eight columns per thread).  A tile is 1024 rows of one column.
-constexpr int kGatherRows = 4;
-template <typename S, bool EXPAND>
-__global__ __launch_bounds__(256) void gather_kernel(const int64_t *__restrict__ idx,
-                                                     const S *__restrict__ x, int64_t ldx,
-                                                     S *__restrict__ y, int64_t ldy, int64_t n_out,
-                                                     int64_t row_tiles, int64_t tiles) {
-    for (int64_t tile = xcd_remap(blockIdx.x, gridDim.x); tile < tiles; tile += gridDim.x) {
-        // (tile indices below 2^32, all but a few, divide as such)
-        const int64_t col = tile >> 32 ? tile / row_tiles : unsigned(tile) / unsigned(row_tiles);
-        const int64_t i0 = (tile - col * row_tiles) * int64_t(256 * kGatherRows) + threadIdx.x;
-        const S *xc = x + col * ldx;
-        S *yc = y + col * ldy;
-        int64_t r[kGatherRows];
+// one column hit its cache lines in any order, so neighbouring workgroups run on one
+// XCD: a column's lines then come from HBM once, into one L2, not once per XCD
+// (70001 of 2^18 rows x 32 complex64: 24 us; 36 with columns spread over all XCDs,
+// 39 with eight columns per thread).
+template <typename S, bool EXPAND, int E>
+__global__ __launch_bounds__(kElemThreads) void gather_kernel(const Rows r,
+                                                              const int64_t *__restrict__ idx,
+                                                              const S *__restrict__ x, int64_t ldx,
+                                                              S *__restrict__ y, int64_t ldy) {
+    const int64_t block = xcd_remap(blockIdx.x, gridDim.x);
+    int64_t at[E];
+    S v[E];
 #pragma unroll
-        for (int e = 0; e < kGatherRows; ++e)
-            r[e] = i0 + e * 256 < n_out ? idx[i0 + e * 256] : -1;
-        S v[kGatherRows] = {};
-#pragma unroll
-        for (int e = 0; e < kGatherRows; ++e)
-            if (r[e] >= 0) v[e] = xc[r[e]];
-#pragma unroll
-        for (int e = 0; e < kGatherRows; ++e)
-            if (EXPAND ? i0 + e * 256 < n_out : r[e] >= 0) yc[i0 + e * 256] = v[e];
-    }
-}
-
-template <typename S>
-__global__ void zero_kernel(S *__restrict__ y, int64_t ldy, int64_t n, int64_t k) {
-    each_group(n, k, [&](int64_t i, int64_t j0, int cols) {
-#pragma unroll
-        for (int c = 0; c < kElemCols; ++c)
-            if (c < cols) y[(j0 + c) * ldy + i] = S{};
+    for (int e = 0; e < E; ++e) v[e] = S(0);
+    each_element<E>(r, block, [&](int e, uint32_t i, uint32_t) { at[e] = idx[i]; });
+    each_element<E>(r, block, [&](int e, uint32_t, uint32_t j) {
+        if (at[e] >= 0) v[e] = x[j * ldx + at[e]];
+    });
+    each_element<E>(r, block, [&](int e, uint32_t i, uint32_t j) {
+        if (EXPAND || at[e] >= 0) y[j * ldy + i] = v[e];
     });
 }
 
-template <typename S>
-__global__ void scatter_kernel(const int64_t *__restrict__ idx, const S *__restrict__ x,
-                               int64_t ldx, S *__restrict__ y, int64_t ldy, int64_t n_in,
-                               int64_t k) {
-    each_group(n_in, k, [&](int64_t i, int64_t j0, int cols) {
-        const int64_t r = idx[i];
-        S v[kElemCols];
-#pragma unroll
-        for (int c = 0; c < kElemCols; ++c)
-            if (c < cols) v[c] = x[(j0 + c) * ldx + i];
-#pragma unroll
-        for (int c = 0; c < kElemCols; ++c)
-            if (c < cols) y[(j0 + c) * ldy + r] = v[c];
-    });
+template <typename S, int E>
+__global__ __launch_bounds__(kElemThreads) void zero_kernel(const Rows r, S *__restrict__ y,
+                                                            int64_t ldy) {
+    each_element<E>(r, blockIdx.x,
+                    [&](int, uint32_t i, uint32_t j) { y[j * ldy + i] = S(0); });
 }
 
-template <typename S>
-__global__ void axpby_kernel(S alpha, const S *x, int64_t ldx, int conj_x, S beta, int use_beta,
-                             S *y, int64_t ldy, int64_t n, int64_t k) {
-    each_group(n, k, [&](int64_t i, int64_t j0, int cols) {
-        S v[kElemCols], w[kElemCols];
-#pragma unroll
-        for (int c = 0; c < kElemCols; ++c)
-            if (c < cols) {
-                v[c] = x[(j0 + c) * ldx + i];
-                if (use_beta) w[c] = y[(j0 + c) * ldy + i];
-            }
-#pragma unroll
-        for (int c = 0; c < kElemCols; ++c)
-            if (c < cols) {
-                S t = v[c];
-                if (conj_x) t = ElemOps<S>::conjv(t);
-                t = ElemOps<S>::mul(alpha, t);
-                if (use_beta) t = ElemOps<S>::add(t, ElemOps<S>::mul(beta, w[c]));
-                y[(j0 + c) * ldy + i] = t;
-            }
+template <typename S, int E>
+__global__ __launch_bounds__(kElemThreads) void scatter_kernel(const Rows r,
+                                                               const int64_t *__restrict__ idx,
+                                                               const S *__restrict__ x, int64_t ldx,
+                                                               S *__restrict__ y, int64_t ldy) {
+    S v[E];
+    int64_t at[E];
+    each_element<E>(r, blockIdx.x, [&](int e, uint32_t i, uint32_t j) {
+        at[e] = idx[i];
+        v[e] = x[j * ldx + i];
+    });
+    each_element<E>(r, blockIdx.x,
+                    [&](int e, uint32_t, uint32_t j) { y[j * ldy + at[e]] = v[e]; });
+}
+
+// y = alpha x + beta y (BETA: beta is not 0, a constant of the kernel, as the compiler
+// got the choice wrong for int8: alpha x + beta y + 1 by v_dot4_u32_u8).
+template <typename S, bool BETA, int E>
+__global__ __launch_bounds__(kElemThreads) void axpby_kernel(const Rows r, S alpha, const S *x,
+                                                             int64_t ldx, int conj_x, S beta,
+                                                             S *y, int64_t ldy) {
+    S v[E], w[E];
+    each_element<E>(r, blockIdx.x, [&](int e, uint32_t i, uint32_t j) {
+        v[e] = x[j * ldx + i];
+        if (BETA) w[e] = y[j * ldy + i];
+    });
+    each_element<E>(r, blockIdx.x, [&](int e, uint32_t i, uint32_t j) {
+        S t = conj_x ? ElemOps<S>::conjv(v[e]) : v[e];
+        t = ElemOps<S>::mul(alpha, t);
+        if (BETA) t = ElemOps<S>::add(t, ElemOps<S>::mul(beta, w[e]));
+        y[j * ldy + i] = t;
     });
 }
 
@@ -212,7 +253,7 @@ static fm_status transpose_launch(int64_t n, int64_t k, const void *src, int64_t
     prof_begin(s, &tok);
     // (a launch for what one grid does not take: loops in the kernel would hold its
     // addresses in registers, 256 of them in place of 55)
-    constexpr int64_t rows = kElemGridX * TR, cols = 65535 * int64_t(TC);
+    constexpr int64_t rows = (int64_t(1) << 22) * TR, cols = 65535 * int64_t(TC);
     for (int64_t i = 0; i < n; i += rows)
         for (int64_t c = 0; c < k; c += cols) {
             const int64_t nn = std::min(n - i, rows), kk = std::min(k - c, cols);
@@ -256,10 +297,11 @@ static fm_status diag_t(int conj_d, int64_t n, const void *d, const void *x, int
                         void *y, int64_t ldy, int64_t k, hipStream_t s) {
     ProfToken tok;
     prof_begin(s, &tok);
-    unsigned nt;
-    const dim3 grid = row_grid(n, k, &nt);
-    hipLaunchKernelGGL(diag_kernel<S>, grid, dim3(nt), 0, s, (const S *)d, (const S *)x,
-                       ldx, (S *)y, ldy, n, k, conj_d);
+    launch_rows<elem_each<S>()>(n, k, [&](auto e, const Rows &r, dim3 grid, int64_t i, int64_t j) {
+        hipLaunchKernelGGL((diag_kernel<S, decltype(e)::value>), grid, dim3(kElemThreads), 0, s, r,
+                           (const S *)d + i, (const S *)x + j * ldx + i, ldx,
+                           (S *)y + j * ldy + i, ldy, conj_d);
+    });
     FM_CHECK_LAUNCH();
     prof_elem(s, &tok, "diag_kernel", sizeof(S), (2.0 * double(n) * double(k) + double(n)) *
                                                      sizeof(S));
@@ -271,10 +313,13 @@ static fm_status gather_any(int64_t n_out, const int64_t *idx, const void *x, in
                           int64_t ldy, int64_t k, hipStream_t s) {
     ProfToken tok;
     prof_begin(s, &tok);
-    const int64_t row_tiles = ceil_div(n_out, 256 * kGatherRows), tiles = row_tiles * k;
-    hipLaunchKernelGGL((gather_kernel<S, EXPAND>), dim3(unsigned(std::min(tiles, kElemGridX))),
-                       dim3(256), 0, s, idx, (const S *)x, ldx, (S *)y, ldy, n_out, row_tiles,
-                       tiles);
+    // (8-byte elements one by one: 8 x 2^20 rows in any order 22 us, four a thread 26)
+    constexpr int E = sizeof(S) <= 4 ? 4 : 1;
+    launch_rows<E>(n_out, k, [&](auto e, const Rows &r, dim3 grid, int64_t i, int64_t j) {
+        hipLaunchKernelGGL((gather_kernel<S, EXPAND, decltype(e)::value>), grid,
+                           dim3(kElemThreads), 0, s, r, idx + i, (const S *)x + j * ldx, ldx,
+                           (S *)y + j * ldy + i, ldy);
+    });
     FM_CHECK_LAUNCH();
     prof_elem(s, &tok, EXPAND ? "expand_kernel" : "gather_kernel", sizeof(S),
               2.0 * double(n_out) * double(k) * sizeof(S) + 8.0 * double(n_out));
@@ -297,14 +342,16 @@ static fm_status scatter_t(int64_t n_in, const int64_t *idx, const void *x, int6
                            int64_t ldy, int64_t n_out, int64_t k, hipStream_t s) {
     ProfToken tok;
     prof_begin(s, &tok);
-    unsigned nt;
-    const dim3 zgrid = row_grid(n_out, k, &nt);
-    hipLaunchKernelGGL(zero_kernel<S>, zgrid, dim3(nt), 0, s, (S *)y, ldy, n_out, k);
-    if (n_in > 0) {
-        const dim3 grid = row_grid(n_in, k, &nt);
-        hipLaunchKernelGGL(scatter_kernel<S>, grid, dim3(nt), 0, s, idx, (const S *)x, ldx,
-                           (S *)y, ldy, n_in, k);
-    }
+    launch_rows<elem_each<S>()>(n_out, k, [&](auto e, const Rows &r, dim3 grid, int64_t i, int64_t j) {
+        hipLaunchKernelGGL((zero_kernel<S, decltype(e)::value>), grid, dim3(kElemThreads), 0, s, r,
+                           (S *)y + j * ldy + i, ldy);
+    });
+    if (n_in > 0)
+        launch_rows<elem_each<S>()>(n_in, k, [&](auto e, const Rows &r, dim3 grid, int64_t i, int64_t j) {
+            hipLaunchKernelGGL((scatter_kernel<S, decltype(e)::value>), grid, dim3(kElemThreads),
+                               0, s, r, idx + i, (const S *)x + j * ldx + i, ldx,
+                               (S *)y + j * ldy, ldy);
+        });
     FM_CHECK_LAUNCH();
     // zero fill and scatter together: every output row written, every input
     // row and index read
@@ -313,21 +360,29 @@ static fm_status scatter_t(int64_t n_in, const int64_t *idx, const void *x, int6
     return FM_SUCCESS;
 }
 
+template <typename S, bool BETA>
+static fm_status axpby_any(int64_t n, int64_t k, const double *alpha, const void *x, int64_t ldx,
+                           int conj_x, const double *beta, void *y, int64_t ldy, hipStream_t s) {
+    ProfToken tok;
+    prof_begin(s, &tok);
+    const S a = ElemOps<S>::from(alpha), b = ElemOps<S>::from(beta);
+    launch_rows<elem_each<S>()>(n, k, [&](auto e, const Rows &r, dim3 grid, int64_t i, int64_t j) {
+        hipLaunchKernelGGL((axpby_kernel<S, BETA, decltype(e)::value>), grid, dim3(kElemThreads),
+                           0, s, r, a, (const S *)x + j * ldx + i, ldx, conj_x, b,
+                           (S *)y + j * ldy + i, ldy);
+    });
+    FM_CHECK_LAUNCH();
+    prof_elem(s, &tok, "axpby_kernel", sizeof(S),
+              (2.0 + BETA) * double(n) * double(k) * sizeof(S));
+    return FM_SUCCESS;
+}
+
 template <typename S>
 static fm_status axpby_t(int64_t n, int64_t k, const double *alpha, const void *x, int64_t ldx,
                          int conj_x, const double *beta, void *y, int64_t ldy, hipStream_t s) {
-    const int use_beta = (beta[0] != 0.0 || beta[1] != 0.0) ? 1 : 0;
-    ProfToken tok;
-    prof_begin(s, &tok);
-    unsigned nt;
-    const dim3 grid = row_grid(n, k, &nt);
-    hipLaunchKernelGGL(axpby_kernel<S>, grid, dim3(nt), 0, s, ElemOps<S>::from(alpha),
-                       (const S *)x, ldx, conj_x, ElemOps<S>::from(beta), use_beta, (S *)y, ldy,
-                       n, k);
-    FM_CHECK_LAUNCH();
-    prof_elem(s, &tok, "axpby_kernel", sizeof(S),
-              (2.0 + use_beta) * double(n) * double(k) * sizeof(S));
-    return FM_SUCCESS;
+    if (beta[0] != 0.0 || beta[1] != 0.0)
+        return axpby_any<S, true>(n, k, alpha, x, ldx, conj_x, beta, y, ldy, s);
+    return axpby_any<S, false>(n, k, alpha, x, ldx, conj_x, beta, y, ldy, s);
 }
 
 }  // namespace fm
@@ -368,7 +423,7 @@ extern "C" fm_status fm_gather_rows(int dtype, int64_t n_out, const int64_t *idx
     if (n_out == 0 || k == 0) return FM_SUCCESS;
     FM_REQUIRE(idx && x && y, FM_ERR_VALUE, "NULL data pointer");
     FM_REQUIRE(ldy >= n_out, FM_ERR_VALUE, "leading dimension below n_out");
-    FM_DISPATCH_ALL(dtype, gather_t, n_out, idx, x, ldx, y, ldy, k, as_stream(stream));
+    FM_DISPATCH_SIZE(dtype, gather_t, n_out, idx, x, ldx, y, ldy, k, as_stream(stream));
 }
 
 extern "C" fm_status fm_expand_rows(int dtype, int64_t n_out, const int64_t *src, const void *x,
@@ -377,7 +432,7 @@ extern "C" fm_status fm_expand_rows(int dtype, int64_t n_out, const int64_t *src
     if (n_out == 0 || k == 0) return FM_SUCCESS;
     FM_REQUIRE(src && x && y, FM_ERR_VALUE, "NULL data pointer");
     FM_REQUIRE(ldy >= n_out, FM_ERR_VALUE, "leading dimension below n_out");
-    FM_DISPATCH_ALL(dtype, expand_t, n_out, src, x, ldx, y, ldy, k, as_stream(stream));
+    FM_DISPATCH_SIZE(dtype, expand_t, n_out, src, x, ldx, y, ldy, k, as_stream(stream));
 }
 
 extern "C" fm_status fm_scatter_rows(int dtype, int64_t n_in, const int64_t *idx, const void *x,
@@ -387,7 +442,7 @@ extern "C" fm_status fm_scatter_rows(int dtype, int64_t n_in, const int64_t *idx
     if (n_out == 0 || k == 0) return FM_SUCCESS;
     FM_REQUIRE(x && y && (idx || n_in == 0), FM_ERR_VALUE, "NULL data pointer");
     FM_REQUIRE(ldy >= n_out && ldx >= n_in, FM_ERR_VALUE, "leading dimension too small");
-    FM_DISPATCH_ALL(dtype, scatter_t, n_in, idx, x, ldx, y, ldy, n_out, k, as_stream(stream));
+    FM_DISPATCH_SIZE(dtype, scatter_t, n_in, idx, x, ldx, y, ldy, n_out, k, as_stream(stream));
 }
 
 extern "C" fm_status fm_axpby(int dtype, int64_t n, int64_t k, const double *alpha, const void *x,
