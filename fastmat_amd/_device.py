@@ -166,14 +166,23 @@ _TRANSPOSE_BYTES = 4 << 20
 def _transpose_bytes(esz, n, k):
     """Size from which the library's transpose of n rows of k elements is the faster
     one.  Measured, own / torch's copy in us:
-    4 and 8 bytes, rows of 8 elements on: 2^18 x 8 float32 6.4 / 7.4, 2^20 x 32 33 / 616,
-      2^18 x 32 float64 19 / 48; shorter rows only when large: 2^20 x 5 float32 8.8 / 7.7,
-      2^18 x 4 float64 6.1 / 5.9, but 2^22 x 2 float32 10 / 14, 2^20 x 4 float64 10 / 17;
-    16 bytes: 2^18 x 32 108 / 76 and 2^20 x 5 74 / 67, but 2^20 x 8 107 / 153;
-    1 byte: 2^22 x 8 38 / 28, but 2^18 x 16 6.8 / 7.6 and 2^22 x 32 121 / 600."""
-    if esz in (4, 8):
-        return _TRANSPOSE_BYTES * (1 if k >= 8 else 8)
-    pays = (k >= 6 and n >= 1 << 20) if esz == 16 else k >= 16
+    - rows that fill its tiles: 2^18 x 8 float32 5.4 / 7.7, 2^20 x 32 33 / 625,
+      2^18 x 32 float64 20 / 49, complex128 46 / 77, 2^20 x 8 complex128 47 / 154;
+    - shorter ones only when large: 2^20 x 5 float32 9.4 / 7.9, 2^18 x 5 complex128
+      13 / 8, but 2^22 x 2 float32 10 / 14, 2^20 x 5 complex128 42 / 67;
+    - small elements by whole tiles of 16 or 32: 2^20 x 12 int8 15 / 11, x 24 33 / 23,
+      but x 16 14 / 20 and x 28 34 / 33; 2^19 x 17 int16 17 / 13, but x 24 19 / 22; or
+      where the columns of torch's copy do not all read a row on the same XCD (row
+      counts that are no multiple of 8192: 700000 x 24 int8 24 / 52) or its L2 does not
+      hold the rows (2^21 x 20 int8 57 / 71);
+    - few rows leave its tiles empty, and torch's copy is in runs of rows:
+      2 x 2500000 float32 97 / 8, 32 x 100000 float64 13 / 11, but 48 x 100000 14 / 18;
+      128 x 100000 complex128 118 / 99, but 256 x 5000 13 / 16."""
+    if esz >= 4:
+        pays = n >= (256 if esz == 16 else 48)
+        return _TRANSPOSE_BYTES * ((1 if k >= 8 else 8) if pays else 1 << 30)
+    pays = n >= 48 and k >= 16 and (k == 16 or k >= (28 if esz == 1 else 20) or
+                                    n % 8192 != 0 or (k >= 20 and n > 1 << 20))
     return _TRANSPOSE_BYTES * (1 if pays else 1 << 30)
 
 
