@@ -76,6 +76,7 @@ _PROTOTYPES = {
     "fm_transpose": (_c_int, [_c_int, _c_i64, _c_i64, _vp, _c_i64, _vp, _c_i64, _vp]),
     "fm_gather_rows": (_c_int, [_c_int, _c_i64, _vp, _vp, _c_i64, _vp, _c_i64, _c_i64, _vp]),
     "fm_expand_rows": (_c_int, [_c_int, _c_i64, _vp, _vp, _c_i64, _vp, _c_i64, _c_i64, _vp]),
+    "fm_invert_index": (_c_int, [_c_int, _c_i64, _vp, _c_i64, _vp, _vp, _vp]),
     "fm_scatter_rows": (_c_int, [_c_int, _c_i64, _vp, _vp, _c_i64, _vp, _c_i64, _c_i64, _c_i64,
                                  _vp]),
     "fm_axpby": (_c_int, [_c_int, _c_i64, _c_i64, ctypes.POINTER(ctypes.c_double), _vp, _c_i64,

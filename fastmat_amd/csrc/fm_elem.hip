@@ -189,6 +189,25 @@ __global__ __launch_bounds__(kElemThreads) void scatter_kernel(const Rows r,
                     [&](int e, uint32_t, uint32_t j) { y[j * ldy + at[e]] = v[e]; });
 }
 
+// A selection's inverse (fm_invert_index): the entries and the flag before, then the
+// selected rows, the largest of equal indices.
+template <typename I>
+__global__ __launch_bounds__(kElemThreads) void invert_fill_kernel(I *__restrict__ inverse,
+                                                                   int64_t n, I *twice) {
+    const int64_t i = blockIdx.x * int64_t(kElemThreads) + threadIdx.x;
+    if (i < n) inverse[i] = -1;
+    if (i == 0) *twice = 0;
+}
+template <typename I>
+__global__ __launch_bounds__(kElemThreads) void invert_kernel(const int64_t *__restrict__ idx,
+                                                              int64_t first, int64_t m,
+                                                              I *inverse, int64_t n, I *twice) {
+    const int64_t i = first + blockIdx.x * int64_t(kElemThreads) + threadIdx.x;
+    if (i >= m) return;
+    const int64_t r = idx[i];
+    if (r >= 0 && r < n && atomicMax(inverse + r, I(i)) >= 0) *twice = 1;
+}
+
 // y = alpha x + beta y (BETA: beta is not 0, a constant of the kernel, as the compiler
 // got the choice wrong for int8: alpha x + beta y + 1 by v_dot4_u32_u8).
 template <typename S, bool BETA, int E>
@@ -386,6 +405,27 @@ static fm_status axpby_t(int64_t n, int64_t k, const double *alpha, const void *
     return axpby_any<S, false>(n, k, alpha, x, ldx, conj_x, beta, y, ldy, s);
 }
 
+template <typename I>
+static fm_status invert_t(int64_t m, const int64_t *idx, int64_t n, void *inverse, void *twice,
+                          hipStream_t s) {
+    constexpr int64_t part = int64_t(1) << 30;  // elements per launch
+    auto grid = [](int64_t count) {
+        return dim3(unsigned(ceil_div(count < part ? count : part, kElemThreads)));
+    };
+    ProfToken tok;
+    prof_begin(s, &tok);
+    for (int64_t i = 0; i < n; i += part)
+        hipLaunchKernelGGL(invert_fill_kernel<I>, grid(n - i), dim3(kElemThreads), 0, s,
+                           (I *)inverse + i, std::min(n - i, part), (I *)twice);
+    for (int64_t i = 0; i < m; i += part)
+        hipLaunchKernelGGL(invert_kernel<I>, grid(m - i), dim3(kElemThreads), 0, s, idx, i, m,
+                           (I *)inverse, n, (I *)twice);
+    FM_CHECK_LAUNCH();
+    prof_elem(s, &tok, "invert_index", sizeof(I),
+              8.0 * double(m) + sizeof(I) * (double(n) + double(m)));
+    return FM_SUCCESS;
+}
+
 }  // namespace fm
 
 using namespace fm;
@@ -434,6 +474,16 @@ extern "C" fm_status fm_expand_rows(int dtype, int64_t n_out, const int64_t *src
     FM_REQUIRE(src && x && y, FM_ERR_VALUE, "NULL data pointer");
     FM_REQUIRE(ldy >= n_out, FM_ERR_VALUE, "leading dimension below n_out");
     FM_DISPATCH_SIZE(dtype, expand_t, n_out, src, x, ldx, y, ldy, k, as_stream(stream));
+}
+
+extern "C" fm_status fm_invert_index(int elem_bytes, int64_t m, const int64_t *idx, int64_t n,
+                                     void *inverse, void *twice, void *stream) {
+    FM_REQUIRE(m >= 0 && n >= 1, FM_ERR_VALUE, "sizes out of range");
+    FM_REQUIRE((idx || m == 0) && inverse && twice, FM_ERR_VALUE, "NULL data pointer");
+    if (elem_bytes == 4) return invert_t<int32_t>(m, idx, n, inverse, twice, as_stream(stream));
+    if (elem_bytes == 8) return invert_t<long long>(m, idx, n, inverse, twice, as_stream(stream));
+    set_error("index inversion: unsupported element size %d", elem_bytes);
+    return FM_ERR_TYPE;
 }
 
 extern "C" fm_status fm_scatter_rows(int dtype, int64_t n_in, const int64_t *idx, const void *x,

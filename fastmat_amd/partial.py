@@ -16,6 +16,18 @@ from .matrix import Hermitian, Matrix
 from .product import Product, select_chain
 
 
+# Matrices whose passes may take the selections (select_chain).
+_FOURIER = (Product, Fourier, Hermitian)
+
+# Selections of vectors up to this length are inverted on the host and go to the device
+# with their indices in one copy; of longer ones the device makes the inverse and the
+# host waits for it.  First forward of a third of the rows of a Fourier matrix, us,
+# host / device / separate passes without an inverse: 1024 points 66 / 84 / 61,
+# 4096 63 / 82 / 66, 16384 82 / 87 / 77, 100003 170 / 112 / 127, 2^18 350 / 132 / 215;
+# rows and columns of 1024 points 78 / 136 / 93.
+_HOST_TABLE = 1 << 14
+
+
 def _check_selection(sel, size, name):
     if sel is None:
         return None
@@ -88,43 +100,79 @@ class Partial(Matrix):
         norms = self._content[0].rowNorms
         return norms if self._rowSelection is None else norms[self._rowSelection]
 
-    def _idx(self, name, sel):
+    def _selections(self):
+        """(name, selection, size of what it selects from) of those given."""
+        M = self._content[0]
+        both = (("r", self._rowSelection, M.numRows), ("c", self._colSelection, M.numCols))
+        return [s for s in both if s[1] is not None]
+
+    def _idx(self, name):
+        """The selection's indices on the device."""
         t = self._dev.get(name)
         if t is None:
-            M = self._content[0]
-            size = M.numRows if name == "r" else M.numCols
-            t = self._dev[name] = D.as_tensor(_device_index(sel, size), np.int64)
+            sel, size = next(s[1:] for s in self._selections() if s[0] == name)
+            t = self._keep(name, D.as_tensor(_device_index(sel, size), np.int64))
         return t
 
-    def _inverse(self, name, sel, dtype=torch.int64):
+    def _keep(self, key, table):
+        """Keep a device table unless there is one: a captured graph holds the address
+        of the one that was there at its capture, which therefore stays."""
+        return self._dev.setdefault(key, table)
+
+    def _upload(self, sels, dtype):
+        """Indices and inverses (_inverse) of the selections to the device, in one
+        copy."""
+        parts, ends, at = [], [], 0
+        for name, sel, size in sels:
+            idx = _device_index(sel, size)
+            inverse = np.full(size + (size & 1), -1, dtype=D.np_dtype(dtype))
+            inverse[idx] = np.arange(len(idx))
+            self._keep("distinct" + name, np.count_nonzero(inverse >= 0) == len(idx))
+            parts += (idx, inverse.view(np.int64))
+            ends.append(at + len(idx))
+            at = ends[-1] + len(parts[-1])
+        t = torch.from_numpy(np.concatenate(parts)).to(D.device())
+        at = 0
+        for (name, _, _), end, inverse in zip(sels, ends, parts[1::2]):
+            self._keep(name, t[at:end])
+            at = end + len(inverse)
+            self._keep((name, dtype), t[end:at].view(dtype))
+
+    def _inverse(self, name, dtype=torch.int64):
         """Row of the selection that lands on each row of the nested matrix's
         operand, -1 for none (the last one of equal indices, as numpy's
         indexed assignment leaves it).  The table is complete before it is kept:
         a later call may run on another stream.  None where it would have to be
         made inside a stream capture, which does not run its kernels."""
-        t = self._dev.get((name, dtype))
-        if t is None and not torch.cuda.is_current_stream_capturing():
-            M = self._content[0]
-            idx = self._idx(name, sel)
-            t = torch.full((M.numRows if name == "r" else M.numCols,), -1, dtype=dtype,
-                           device=idx.device)
-            t.scatter_reduce_(0, idx, torch.arange(idx.numel(), dtype=dtype, device=idx.device),
-                              "amax")
-            torch.cuda.current_stream(idx.device).synchronize()
-            self._dev[name, dtype] = t
-        return t
+        if (name, dtype) not in self._dev and not torch.cuda.is_current_stream_capturing():
+            # (the transform's passes take both, an expansion its own)
+            sels = [s for s in self._selections() if dtype == torch.int32 or s[0] == name]
+            if max(s[2] for s in sels) <= _HOST_TABLE:
+                self._upload(sels, dtype)
+            else:
+                self._invert(sels, dtype)
+        return self._dev.get((name, dtype))
 
-    def _distinct(self, name, sel):
-        """True when no element is selected twice (counted on the device, once:
-        32 us on 2^18 elements, 190 in numpy); False inside a stream capture
+    def _invert(self, sels, dtype):
+        """Inverses of the selections by the device, with one wait for all of them."""
+        t = torch.empty(sum(size for _, _, size in sels) + len(sels), dtype=dtype,
+                        device=D.device())
+        tables, at = [], len(sels)
+        for q, (name, sel, size) in enumerate(sels):
+            tables.append(t[at:at + size])
+            _lib.call("fm_invert_index", t.element_size(), len(sel), _lib.ptr(self._idx(name)),
+                      size, _lib.ptr(tables[-1]), _lib.ptr(t[q:]), D.stream())
+            at += size
+        for twice, table, (name, _, _) in zip(t[:len(sels)].tolist(), tables, sels):
+            self._keep((name, dtype), table)
+            self._keep("distinct" + name, not twice)
+
+    def _distinct(self, name):
+        """True when no element is selected twice; False inside a stream capture
         where it is not known yet."""
-        d = self._dev.get("distinct" + name)
-        if d is None:
-            t = self._inverse(name, sel, torch.int32)
-            if t is None or torch.cuda.is_current_stream_capturing():
-                return False
-            d = self._dev["distinct" + name] = int(torch.count_nonzero(t >= 0)) == len(sel)
-        return d
+        if "distinct" + name not in self._dev:
+            self._inverse(name, torch.int32)
+        return self._dev.get("distinct" + name, False)
 
     def _selected(self, X, adjoint):
         """The product with both selections inside the passes of the nested
@@ -132,7 +180,7 @@ class Partial(Matrix):
         name an element twice for the result, empty ones, and a capture before
         the tables are there."""
         M = self._content[0]
-        if type(M) not in (Product, Fourier, Hermitian) or X.shape[0] == 0:
+        if type(M) not in _FOURIER or X.shape[0] == 0:
             return None
         ins, outs = ("c", self._colSelection), ("r", self._rowSelection)
         if adjoint:
@@ -142,15 +190,11 @@ class Partial(Matrix):
             return None
 
         def tables():
-            for name, sel in (ins, outs):
-                if sel is not None:
-                    self._idx(name, sel)  # an index out of range is an error here
-            if outs[1] is not None and not self._distinct(*outs):
-                return None
-            made = [None if sel is None else self._inverse(name, sel, torch.int32)
+            made = [None if sel is None else self._inverse(name, torch.int32)
                     for name, sel in (ins, outs)]
-            return made if all(s is None or t is not None
-                               for t, (_, s) in zip(made, (ins, outs))) else None
+            if any(s is not None and t is None for t, (_, s) in zip(made, (ins, outs))):
+                return None
+            return made if outs[1] is None or self._distinct(outs[0]) else None
         return select_chain(M, X, adjoint, ins[1] is not None, outs[1] is not None, tables,
                             self.numCols if adjoint else self.numRows)
 
@@ -159,9 +203,9 @@ class Partial(Matrix):
         Y = D.empty(k, n_full, X.dtype)
         if n == 0:
             return Y.zero_()
-        inverse = self._inverse(name, sel)
+        inverse = self._inverse(name)
         if inverse is None:  # (a capture that no call of this direction came before)
-            _lib.call("fm_scatter_rows", D.fm_type(X.dtype), n, _lib.ptr(self._idx(name, sel)),
+            _lib.call("fm_scatter_rows", D.fm_type(X.dtype), n, _lib.ptr(self._idx(name)),
                       _lib.ptr(X), n, _lib.ptr(Y), n_full, n_full, k, D.stream())
         else:
             _lib.call("fm_expand_rows", D.fm_type(X.dtype), n_full, _lib.ptr(inverse),
@@ -172,7 +216,7 @@ class Partial(Matrix):
         k, n = X.shape
         m = len(sel)
         Y = D.empty(k, m, X.dtype)
-        _lib.call("fm_gather_rows", D.fm_type(X.dtype), m, _lib.ptr(self._idx(name, sel)),
+        _lib.call("fm_gather_rows", D.fm_type(X.dtype), m, _lib.ptr(self._idx(name)),
                   _lib.ptr(X), n, _lib.ptr(Y), m, k, D.stream())
         return Y
 

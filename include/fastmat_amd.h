@@ -416,6 +416,11 @@ fm_status fm_gather_rows(int dtype, int64_t n_out, const int64_t *idx,
  * zero-padded scatter from its inverse index, one write per row. */
 fm_status fm_expand_rows(int dtype, int64_t n_out, const int64_t *src, const void *x,
                          int64_t ldx, void *y, int64_t ldy, int64_t k, void *stream);
+/* Inverse of a selection: inverse[idx[i]] = i for i < m (the largest i of equal
+ * indices), -1 elsewhere, for n entries; *twice = 1 when two indices are equal, else 0.
+ * idx: device int64, within [0, n); inverse and twice: elements of 4 or 8 bytes. */
+fm_status fm_invert_index(int elem_bytes, int64_t m, const int64_t *idx, int64_t n,
+                          void *inverse, void *twice, void *stream);
 /* y = 0 (n_out rows); y[idx[i],:] = x[i,:] for i < n_in (Partial's
  * zero-padded scatter, Partial.pyx:270-276). */
 fm_status fm_scatter_rows(int dtype, int64_t n_in, const int64_t *idx,
