@@ -142,13 +142,13 @@ class Fourier(Matrix):
                   None if ws is None else _lib.ptr(ws), need.value, D.stream())
         return Y
 
-    def _diag_ok(self, X):
-        """True when diagonals can run inside the transform of X: a
-        power-of-two order (Bluestein's chirps take their place otherwise) and
-        data that is already of the compute type."""
-        return (self._order & (self._order - 1) == 0 and
-                D.np_dtype(X.dtype) == self.compute_dtype(X.dtype) and
-                D.promote(X.dtype, self._minType) == D.np_dtype(X.dtype))
+    def _diag_ok(self, dtype):
+        """True when diagonals can run inside the transform of data of the torch
+        type: a power-of-two order (Bluestein's chirps take their place otherwise)
+        and the compute type."""
+        dt = D.np_dtype(dtype)
+        return (self._order & (self._order - 1) == 0 and dt == self.compute_dtype(dtype) and
+                D.promote(dtype, self._minType) == dt)
 
     def _run_diag(self, X, adjoint, pre, post):
         """diag(post) F diag(pre) X, or its conjugates around F^H (pre, post:
@@ -165,18 +165,18 @@ class Fourier(Matrix):
                   need.value, D.stream())
         return Y
 
-    def _select_ok(self, X):
-        """True when the passes over X can read and store selected elements: data
-        of the compute type, and a transform whose first and last passes are
-        plain ones of the lengths the selecting kernels have (a one-pass chirp
-        transform has one spectrum pass; four-step passes up to 2048 points)."""
-        if (D.np_dtype(X.dtype) != self.compute_dtype(X.dtype) or
-                D.promote(X.dtype, self._minType) != D.np_dtype(X.dtype)):
+    def _select_ok(self, dtype):
+        """True when the passes over data of the torch type can read and store
+        selected elements: the compute type, and a transform whose first and last
+        passes are plain ones of the lengths the selecting kernels have (a one-pass
+        chirp transform has one spectrum pass; four-step passes up to 2048 points)."""
+        dt = D.np_dtype(dtype)
+        if dt != self.compute_dtype(dtype) or D.promote(dtype, self._minType) != dt:
             return False
         n = self._order
         if n & (n - 1) == 0:
             return n <= 1 << 22
-        one_pass = 8192 if X.dtype == torch.complex64 else 4096
+        one_pass = 8192 if dtype == torch.complex64 else 4096
         return one_pass < 2 * n - 1 <= 1 << 22
 
     def _run_select(self, X, adjoint, pre, post, in_index, out_index, m):

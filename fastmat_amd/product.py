@@ -105,7 +105,7 @@ def _fourier_with_diags(factors, i, X, adjoint):
         return None
     F, flip = _as_fourier(factors[f])
     post = factors[f + 1] if f + 1 < len(factors) and type(factors[f + 1]) is Diag else None
-    if F is None or (pre is None and post is None) or not _diags_ok(F, X, pre, post):
+    if F is None or (pre is None and post is None) or not _diags_ok(F, X.dtype, pre, post):
         return None
     # the transform conjugates its tables when it is an adjoint one; a Diag's
     # adjoint is its conjugate
@@ -125,10 +125,11 @@ def _diag_tables(dt, conj, *diags):
     return tables
 
 
-def _diags_ok(F, X, *diags):
-    """True when the Diag factors (or None) can run inside F's transform of X."""
-    dt = D.np_dtype(X.dtype)
-    return F._diag_ok(X) and all(
+def _diags_ok(F, dtype, *diags):
+    """True when the Diag factors (or None) can run inside F's transform of data of
+    the torch type."""
+    dt = D.np_dtype(dtype)
+    return F._diag_ok(dtype) and all(
         d is None or (D.promote(dt, d.dtype) == dt and D.promote(dt, d._minType) == dt)
         for d in diags)
 
@@ -155,33 +156,32 @@ def select_chain(M, X, adjoint, select_in, select_out, tables, m):
     post = factors[f + 1] if f + 1 < len(factors) and type(factors[f + 1]) is Diag else None
     if F is None or f + 1 + (post is not None) != len(factors):
         return None
+    # the type that the transform takes, by M's rules and (real data becomes complex) its
+    # own; the data follows once it is to run here
     t = D.input_type(X.dtype, M._minType, M.dtype, M._widenInputDatatype)
-    if X.dtype is not t:
-        X = X.to(t)
     if type(M) is Product:
-        dt = D.promote(X.dtype, M.dtype)
-        if D.np_dtype(X.dtype) != dt:
-            X = X.to(D.torch_dtype(dt))
+        t = D.torch_dtype(D.promote(t, M.dtype))
     if pre is None:
-        # (the transform's own type rules: real data becomes complex)
-        X = X.to(D.torch_dtype(F.compute_dtype(
-            D.input_type(X.dtype, F._minType, F.dtype, F._widenInputDatatype))))
-    if not F._select_ok(X):
+        t = D.torch_dtype(F.compute_dtype(
+            D.input_type(t, F._minType, F.dtype, F._widenInputDatatype)))
+    if not F._select_ok(t):
         return None
-    inside = _diags_ok(F, X, pre, post)
+    inside = _diags_ok(F, t, pre, post)
     if not inside and ((pre is not None and select_in) or (post is not None and select_out)):
         return None
     inverse = adjoint != flip
-    diags = _diag_tables(D.np_dtype(X.dtype), inverse != adjoint,
+    diags = _diag_tables(D.np_dtype(t), inverse != adjoint,
                          *((pre, post) if inside else (None, None)))
     index = None if diags is None else tables()
     if index is None:
         return None
+    if X.dtype is not t:
+        X = X.to(t)
     if scalar:
         X = M._prep(X, adjoint and np.iscomplexobj(M._scalar))
     if pre is not None and not inside:
         X = pre._apply(X, adjoint)
-        if not F._select_ok(X):
+        if not F._select_ok(X.dtype):
             return None
     Y = F._run_select(X, inverse, *diags, *index, m)
     if Y is not None and post is not None and not inside:
