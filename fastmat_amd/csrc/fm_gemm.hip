@@ -364,16 +364,19 @@ static int cu_count() {
 
 template <typename S, bool XC, bool AK, int FM, int FN, int WM, int WN, int WK,
           typename Off = uint32_t>
-static fm_status direct_launch(const DirectArgs<S> &g, hipStream_t stream) {
-    constexpr int TM = 16 * FM * WM, TN = (XC ? 8 : 16) * FN * WN;
+static fm_status direct_launch(DirectArgs<S> g, hipStream_t stream) {
+    constexpr int TM = 16 * FM * WM, TN = (XC ? 8 : 16) * FN * WN, NT = 64 * WM * WN * WK;
     constexpr size_t lds = WK > 1 ? size_t(WM) * WN * WK * FN * 4 * FM * 64 * sizeof(S) : 0;
     static_assert(lds <= 64 * 1024, "K split's partial sums");
     const int64_t tiles = ceil_div(g.M, TM) * ceil_div(g.NC, TN);
-    FM_REQUIRE(tiles < (int64_t(1) << 31), FM_ERR_VALUE, "dense product too large for one launch");
     ProfToken tok;
     prof_begin(stream, &tok);
-    hipLaunchKernelGGL((gemm_direct_kernel<S, Off, XC, AK, FM, FN, WM, WN, WK>), dim3(unsigned(tiles)),
-                       dim3(64 * WM * WN * WK), lds, stream, g);
+    // (a launch of 2^32 threads or more runs what is left of that number)
+    constexpr int64_t part = (int64_t(1) << 31) / NT;
+    for (g.tile0 = 0; g.tile0 < tiles; g.tile0 += part)
+        hipLaunchKernelGGL((gemm_direct_kernel<S, Off, XC, AK, FM, FN, WM, WN, WK>),
+                           dim3(unsigned(std::min(tiles - g.tile0, part))), dim3(NT), lds, stream,
+                           g);
     FM_CHECK_LAUNCH();
     if (tok.active) {
         const double e = double(sizeof(S)), xs = XC ? 2.0 : 1.0;

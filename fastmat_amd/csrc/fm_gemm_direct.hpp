@@ -53,6 +53,7 @@ template <typename S> struct DirectArgs {
     S *Y;
     int64_t ldy;
     int conj_a;  // complex A: multiply by its conjugate
+    int64_t tile0;  // the launch's first tile
 };
 
 typedef float dg_f4 __attribute__((ext_vector_type(4)));
@@ -163,7 +164,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void gemm_direct_kernel(
     const int r = lane & 15, h = lane >> 4;
     const int wk = wave % WK, wn = (wave / WK) % WN, wm = wave / (WK * WN);
     const int64_t tiles_n = ceil_div(g.NC, TN);
-    const int64_t tile = xcd_remap(blockIdx.x, gridDim.x);
+    const int64_t tile = g.tile0 + xcd_remap(blockIdx.x, gridDim.x);
     const int64_t tm = tile / tiles_n, tn = tile - tm * tiles_n;
     const int64_t i0 = tm * TM + wm * (16 * FM), c0 = tn * TN + wn * CW;
     const int64_t steps = ceil_div(g.K, BK);
