@@ -426,6 +426,15 @@ static fm_status direct_pick(const DirectArgs<S> &g, hipStream_t stream) {
     if (reach >= 4294967296.0 || xreach >= 4294967296.0)
         return direct_launch<S, XC, AK, 1, X2, 1, 1, 8, uint64_t>(g, stream);
     if constexpr (XC) {
+        // short sums with a wave for every SIMD: what bounds them is Y, and a K split's
+        // waves wait for its partial sums (us, M x K x NC, before the shapes below, with
+        // them / this): 129 x 4 x 60000 43, 57 / 25; 300 x 200 x 60000 337, 181 / 154;
+        // 100 x 400 x 60000 139 / 123, but x 20000 (1250 tiles) 55 / 58; 1000 x 1000 x
+        // 3000 247, 111 / 137; a 16-row tile holds fewer rows better: 8 x 300 x 60000
+        // 27 / 48, 20 x 140 x 60000 34 / 29
+        const int64_t waves = ceil_div(g.M, 64) * ceil_div(g.NC, 32);
+        if (g.M > 16 && g.K <= 512 && waves >= (g.K <= 256 ? 4 : 8) * int64_t(cost.ncu))
+            return direct_launch<S, XC, AK, 4, 4, 1, 1, 1>(g, stream);
         const double a = 2 * cost(128, 64, 1.0), b = 2 * cost(64, 32, AK ? 1.05 : 1.1),
                      e = 2 * cost(64, 16, AK ? 1.2 : 1.03), d = 2 * cost(16, 16, 2.4);
         if (a <= b && a <= e && a <= d) return direct_launch<S, XC, AK, 4, 4, 2, 2, 1>(g, stream);

@@ -348,6 +348,19 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2) void gemm_direct_kernel(
             const int64_t i = i0 + 16 * V * u + V * r;
             if constexpr (XC) {
                 S *y = g.Y + 2 * (c * g.ldy + i);
+                if constexpr (V > 1) {
+                    if (i + V <= g.M) {
+                        S t[2 * V];
+#pragma unroll
+                        for (int e = 0; e < V; ++e) {
+                            t[2 * e] = re[u * V + e];
+                            t[2 * e + 1] = im[u * V + e];
+                        }
+#pragma unroll
+                        for (int e = 0; e < 2 * V; e += KS) store16(y + e, t + e);
+                        continue;
+                    }
+                }
 #pragma unroll
                 for (int e = 0; e < V; ++e)
                     if (i + e < g.M) {
