@@ -3,17 +3,16 @@
 //
 // Method (written from the published Stockham autosort formulation): a
 // length-N transform (N = 2^LOGN, compile-time) is split into S stages of
-// radix 2^bits(s) <= E, E = 32 (complex64) or 16 (complex128) elements per
-// thread.  Stage with radix R and sub-length p: butterfly i in [0, N/R) takes
+// radix 2^bits(s) <= E, E = 4 to 32 elements per thread by the pass's shape (see
+// PassShape).  Stage with radix R and sub-length p: butterfly i in [0, N/R) takes
 // X[i + r N/R], multiplies input r by W_{pR}^{r k} (k = i mod p), runs an
 // R-point DFT in registers and produces Y[(i - k) R + k + r p]; outputs come
 // out in natural order.  Stage 0 loads its inputs straight from HBM, the last
 // stage stores straight to HBM, and the S-1 exchanges in between go through a
-// padded LDS tile (one spare slot per 32 elements).  1024 = 32 x 32 needs one
-// exchange.
+// padded LDS tile (see tile_row).  1024 = 32 x 32 needs one exchange.
 //
-// Tile: B = 256 * E / N consecutive sequences s = o*J + j of an (O x J)
-// sequence space (512 threads for the largest N).  Element n of sequence
+// Tile: B = threads * E / N consecutive sequences s = o*J + j of an (O x J)
+// sequence space.  Element n of sequence
 // (o, j) is read at  x[o*in_os + j*in_js + n*in_ns]  and written at
 // y[o*out_os + j*out_js + n*out_ns]; this one addressing form covers
 // contiguous columns, the strided and the transposed sides of the four-step
@@ -721,7 +720,7 @@ struct PlainMid {};
 
 // Everything after the stage-0 loads of one tile: conj / pre-multiply, the
 // transform (conv: forward, spectrum, inverse), twiddle / post-multiply and
-// the stores.  `lds` holds B * (N + N/32 + 1) elements.
+// the stores.  `lds` holds B * tile_row<T>(LOGN, LOGB) elements (tile_lds_bytes).
 template <typename T, int LOGN, int NT, bool CONV, bool I32 = false, int LE = -1,
           typename EP = PlainStore, typename MP = PlainMid>
 __device__ __forceinline__ void fft_tile_compute(const TileArgs<T> &a, int64_t tile, cpx<T> *v,
