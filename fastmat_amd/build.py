@@ -12,6 +12,7 @@ import os
 import shutil
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -40,25 +41,24 @@ def flags():
 
 
 def build(verbose=False, jobs=8):
-    srcs = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
+    # largest source first (fm_batch.hip compiles longest), a new one as one ends
+    srcs = sorted(glob.glob(os.path.join(CSRC, "*.hip")), key=lambda s: (-os.path.getsize(s), s))
     objdir = os.path.join(HERE, "_build")
     os.makedirs(objdir, exist_ok=True)
     cc = hipcc()
-    procs = []
-    objs = []
-    for src in srcs:
+
+    def compile_one(src):
         obj = os.path.join(objdir, os.path.basename(src) + ".o")
-        objs.append(obj)
         cmd = [cc] + flags() + ["-c", src, "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)
-        procs.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE,
-                                            stderr=subprocess.STDOUT)))
-        if len(procs) >= jobs:
-            _drain(procs)
-    _drain(procs)
+        return obj, src, subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)
+
+    with ThreadPoolExecutor(jobs) as pool:
+        done = list(pool.map(compile_one, srcs))
+    _check(done)
     tmp = OUT + ".tmp"
-    cmd = [cc] + flags() + ["-shared", "-o", tmp] + objs
+    cmd = [cc] + flags() + ["-shared", "-o", tmp] + sorted(obj for obj, _, _ in done)
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
@@ -66,12 +66,10 @@ def build(verbose=False, jobs=8):
     return OUT
 
 
-def _drain(procs):
+def _check(done):
     errors = []
-    while procs:
-        src, p = procs.pop(0)
-        out, _ = p.communicate()
-        text = out.decode(errors="replace")
+    for _, src, p in done:
+        text = p.stdout.decode(errors="replace")
         # drop the host pass's notice about the device-only target feature
         lines = [l for l in text.splitlines() if "packed-fp32-ops" not in l
                  and "is not a recognized feature" not in l]
